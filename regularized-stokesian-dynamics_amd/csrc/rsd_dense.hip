@@ -316,16 +316,23 @@ __device__ __forceinline__ void wt_publish(int* flag, int gen) {
 __device__ __forceinline__ void wt_seen() { __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront"); }
 
 // A 64x64 tile of the factorization (published by another workgroup) into
-// LDS by direct 16-byte loads at agent scope, past any stale cached copy.
-__device__ __forceinline__ void stage_tile(const double* __restrict__ src, size_t ld, double* __restrict__ dst) {
+// LDS by direct 16-byte loads at agent scope, past any stale cached copy:
+// a wave's u-th load (of 8) moves columns 16 wave + 2u and 16 wave + 2u + 1;
+// at: the lane's offset into the tile (stage_at), the same for every u.
+__device__ __forceinline__ unsigned stage_at(int ld) {
   const int tid = opaque_tid(), lane = tid & 63, wave = tid >> 6;
+  return (unsigned)((16 * wave + (lane >> 5)) * ld + 2 * ((lane & 31) ^ ((lane >> 5) << 3)));
+}
+__device__ __forceinline__ void stage_load(const double* p, int ld, unsigned at, int u, double* dst) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(p + (size_t)(2 * u) * ld + at),
+                                   (__attribute__((address_space(3))) void*)(dst + (wave * 8 + u) * 128), 16, 0,
+                                   kCpolSc1);
+}
+__device__ __forceinline__ void stage_tile(const double* src, int ld, double* dst) {
+  const unsigned at = stage_at(ld);
 #pragma unroll
-  for (int q = 0; q < 8; ++q) {
-    const int chunk = wave * 8 + q;
-    const int c = 2 * chunk + (lane >> 5), pr = (lane & 31) ^ ((c & 1) << 3);
-    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src + (size_t)c * ld + 2 * pr),
-                                     (__attribute__((address_space(3))) void*)(dst + chunk * 128), 16, 0, kCpolSc1);
-  }
+  for (int u = 0; u < 8; ++u) stage_load(src, ld, at, u, dst);
 }
 
 // element (m, c) of a staged tile
@@ -1038,53 +1045,6 @@ __device__ __forceinline__ void tile_store_direct_t(const v4d (&acc)[2][2], doub
                  acc[bm][bn][v]);
 }
 
-// One term of a tile's accumulation: tiles (i,k) and (j,k) (one tile when
-// i == j) staged in LDS, (i,k) first.
-__device__ __forceinline__ void stage_term(const double* __restrict__ A, size_t ld, int i, int j, int k,
-                                           double* __restrict__ dst) {
-  stage_tile(A + 64 * i + (size_t)(64 * k) * ld, ld, dst);
-  if (i != j) stage_tile(A + 64 * j + (size_t)(64 * k) * ld, ld, dst + 4096);
-}
-
-// Two 64x64 tiles from anywhere (the first at dst, the second at dst + 4096).
-__device__ __forceinline__ void stage_pair(const double* p1, size_t ld1, const double* p2, size_t ld2,
-                                           double* __restrict__ dst) {
-  stage_tile(p1, ld1, dst);
-  stage_tile(p2, ld2, dst + 4096);
-}
-
-// nacc += L_ik L_jk^T (nacc: the tile negated) from a staged term (cur), the
-// next term's loads (into nxt, when pre) in flight meanwhile.  All 16 steps'
-// operands are read into registers first, so that the LDS reads run ahead of
-// the MFMAs that use them instead of each step waiting for its own reads,
-// and so that they precede the direct-to-LDS loads of the next term: LDS
-// reads issued after those loads would wait for them to land.
-__device__ __forceinline__ void term_product(v4d (&nacc)[2][2], const double* __restrict__ A, size_t ld, int i, int j,
-                                             int knext, bool pre, const double* __restrict__ cur,
-                                             double* __restrict__ nxt) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
-  const double* cb = cur + (i == j ? 0 : 4096);
-  const int m = lane & 15, kq = lane >> 4;
-  double a0[16], a1[16], b0[16], b1[16];
-#pragma unroll
-  for (int st = 0; st < 16; ++st) {
-    const int kr = 4 * st + kq;
-    a0[st] = cur[staged(wm + m, kr)];
-    a1[st] = cur[staged(wm + 16 + m, kr)];
-    b0[st] = cb[staged(wn + m, kr)];
-    b1[st] = cb[staged(wn + 16 + m, kr)];
-  }
-  if (pre) stage_term(A, ld, i, j, knext, nxt);
-#pragma unroll
-  for (int st = 0; st < 16; ++st) {
-    nacc[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0[st], b0[st], nacc[0][0], 0, 0, 0);
-    nacc[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0[st], b1[st], nacc[0][1], 0, 0, 0);
-    nacc[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1[st], b0[st], nacc[1][0], 0, 0, 0);
-    nacc[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1[st], b1[st], nacc[1][1], 0, 0, 0);
-  }
-}
-
 __device__ __forceinline__ void tile_negate(v4d (&acc)[2][2]) {
 #pragma unroll
   for (int bm = 0; bm < 2; ++bm)
@@ -1092,147 +1052,208 @@ __device__ __forceinline__ void tile_negate(v4d (&acc)[2][2]) {
     for (int bn = 0; bn < 2; ++bn) acc[bm][bn] = -acc[bm][bn];
 }
 
-// acc -= sum_{k < kend} L_ik L_jk^T, each term once tiles (i,k), (j,k) are
-// published.  Terms go through two LDS buffers of 2 x 64 x 64 doubles: the
-// loads of term k+1 overlap the products of term k whenever term k+1 is
-// already published when term k starts.
-__device__ __forceinline__ void tile_accumulate(v4d (&acc)[2][2], const double* __restrict__ A, int ld, int nt, int i,
-                                                int j, int kend, const int* flags, int gen, int* err, double* smem,
-                                                int* rec, int who) {
-  const int tid = threadIdx.x;
-  __shared__ int kready_s;
-  int kready = 0;
-  // wait for term k, then take every later term that is already published
-  // too: one barrier per batch, not per term
-  auto ready = [&](int k) {
-    if (tid == 0) {
-      wait_flag(&flags[i + nt * k], gen, err, rec, who, i + nt * k);
-      if (i != j) wait_flag(&flags[j + nt * k], gen, err, rec, who, j + nt * k);
-      int kk = k + 1;
-      while (kk < kend && __hip_atomic_load(&flags[i + nt * kk], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gen &&
-             __hip_atomic_load(&flags[j + nt * kk], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gen)
-        ++kk;
-      kready_s = kk;
-    }
-    __syncthreads();
-    kready = kready_s;
-    wt_seen();
-  };
-  if (kend <= 0) return;
-  tile_negate(acc);  // the terms add to the negated tile (exact: negation commutes with rounding)
-  ready(0);
-  stage_term(A, (size_t)ld, i, j, 0, smem);
-  __builtin_amdgcn_s_waitcnt(kWaitVm0);
-  __syncthreads();
-  for (int k = 0; k < kend; ++k) {
-    double* cur = smem + (k & 1) * 8192;
-    double* nxt = smem + ((k + 1) & 1) * 8192;
-    const bool more = k + 1 < kend, pre = more && k + 1 < kready;
-    term_product(acc, A, (size_t)ld, i, j, k + 1, pre, cur, nxt);
-    if (more && !pre) {
-      ready(k + 1);
-      stage_term(A, (size_t)ld, i, j, k + 1, nxt);
-    }
-    __builtin_amdgcn_s_waitcnt(kWaitVm0);
-    __syncthreads();
-  }
-  tile_negate(acc);
+// The MFMA operands of eight 4-deep steps of a staged pair (T1 at the buffer,
+// T2 4096 doubles on), and their products.  Half h of a term is steps 8h..8h+7.
+struct HalfOps {
+  double a0[8], a1[8], b0[8], b1[8];
+};
+// where this lane's operands of an even step (T1's two row blocks, T2's) lie
+// in a buffer; odd steps' columns have the same parity, so one offset serves
+// all steps: step st is 256 st doubles on
+struct HalfAt {
+  int a0, a1, b0, b1;
+};
+__device__ __forceinline__ HalfAt half_at() {
+  const int tid = opaque_tid(), lane = tid & 63, wave = tid >> 6;
+  const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32, m = lane & 15, kq = lane >> 4;
+  return {staged(wm + m, kq), staged(wm + 16 + m, kq), 4096 + staged(wn + m, kq), 4096 + staged(wn + 16 + m, kq)};
 }
-
-// nacc += T1 T2^T for a staged pair (T1 at cur, T2 at cur + 4096); stage()
-// issues the next pair's loads into nxt (when pre), after this pair's
-// operands are read (as in term_product).
-template <class Stage>
-__device__ __forceinline__ void pair_product(v4d (&nacc)[2][2], bool pre, const double* __restrict__ cur,
-                                             Stage&& stage) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
-  const double* cb = cur + 4096;
-  const int m = lane & 15, kq = lane >> 4;
-  double a0[16], a1[16], b0[16], b1[16];
-#pragma unroll
-  for (int st = 0; st < 16; ++st) {
-    const int kr = 4 * st + kq;
-    a0[st] = cur[staged(wm + m, kr)];
-    a1[st] = cur[staged(wm + 16 + m, kr)];
-    b0[st] = cb[staged(wn + m, kr)];
-    b1[st] = cb[staged(wn + 16 + m, kr)];
+__device__ __forceinline__ void half_read(HalfOps& o, const HalfAt& at, int u, int h, const double* buf) {
+  const double* b = buf + 256 * (8 * h + u);
+  o.a0[u] = b[at.a0];
+  o.a1[u] = b[at.a1];
+  o.b0[u] = b[at.b0];
+  o.b1[u] = b[at.b1];
+}
+__device__ __forceinline__ void half_mfma(v4d (&nacc)[2][2], const HalfOps& o, int u) {
+  nacc[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(o.a0[u], o.b0[u], nacc[0][0], 0, 0, 0);
+  nacc[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(o.a0[u], o.b1[u], nacc[0][1], 0, 0, 0);
+  nacc[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(o.a1[u], o.b0[u], nacc[1][0], 0, 0, 0);
+  nacc[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(o.a1[u], o.b1[u], nacc[1][1], 0, 0, 0);
+}
+// the tiles of one term
+struct TermSrc {
+  const double *p1, *p2;
+  int ld1, ld2;
+};
+// one half's products.  Between each step's MFMAs go one step's reads of the
+// next half's operands (half hnext of the term at rd) and, with ST, two loads
+// of a later term's tiles t1, t2 into wr: bunched in front, either would leave
+// the matrix cores idle behind them (the fence keeps them where they are).
+// The restrict pointers tell the compiler that the reads of rd may pass the
+// loads into wr.
+template <bool ST>
+__device__ __forceinline__ void half_product(v4d (&nacc)[2][2], const HalfOps& use, HalfOps& next, const HalfAt& at,
+                                             int hnext, const double* __restrict__ rd, const double* __restrict__ t1,
+                                             int ld1, const double* __restrict__ t2, int ld2,
+                                             double* __restrict__ wr) {
+  unsigned at1 = 0, at2 = 0;
+  if (ST) {
+    at1 = stage_at(ld1);
+    at2 = stage_at(ld2);
   }
-  if (pre) stage();
 #pragma unroll
-  for (int st = 0; st < 16; ++st) {
-    nacc[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0[st], b0[st], nacc[0][0], 0, 0, 0);
-    nacc[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0[st], b1[st], nacc[0][1], 0, 0, 0);
-    nacc[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1[st], b0[st], nacc[1][0], 0, 0, 0);
-    nacc[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1[st], b1[st], nacc[1][1], 0, 0, 0);
+  for (int u = 0; u < 8; ++u) {
+    half_read(next, at, u, hnext, rd);
+    if (ST) {
+      stage_load(t1, ld1, at1, u, wr);
+      stage_load(t2, ld2, at2, u, wr + 4096);
+    }
+    half_mfma(nacc, use, u);
+    __builtin_amdgcn_sched_barrier(0);
   }
 }
 
-// acc -= sum_{kbeg <= k < kend} T1_k T2_k^T, with src(k, p1, ld1, p2, ld2, f1,
-// f2) naming term k's two tiles and their flags (indices into flags); each
-// term once both flags are published (as tile_accumulate).
-template <class Src>
-__device__ __forceinline__ void pair_accumulate(v4d (&acc)[2][2], int kbeg, int kend, Src&& src, const int* flags,
-                                                int gen, int* err, double* smem, int* rec, int who) {
-  const int tid = threadIdx.x;
-  __shared__ int kready_x;
-  int kready = kbeg;
-  auto published = [&](int k) {
-    const double *p1, *p2;
-    size_t l1, l2;
-    int f1, f2;
-    src(k, p1, l1, p2, l2, f1, f2);
-    return __hip_atomic_load(&flags[f1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gen &&
-           __hip_atomic_load(&flags[f2], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gen;
-  };
-  auto ready = [&](int k) {
-    if (tid == 0) {
-      const double *p1, *p2;
-      size_t l1, l2;
-      int f1, f2;
-      src(k, p1, l1, p2, l2, f1, f2);
-      wait_flag(&flags[f1], gen, err, rec, who, f1);
-      wait_flag(&flags[f2], gen, err, rec, who, f2);
-      int kk = k + 1;
-      while (kk < kend && published(kk)) ++kk;
-      kready_x = kk;
-    }
-    __syncthreads();
-    kready = kready_x;
-    wt_seen();
-  };
-  auto stage = [&](int k, double* dst) {
-    const double *p1, *p2;
-    size_t l1, l2;
-    int f1, f2;
-    src(k, p1, l1, p2, l2, f1, f2);
-    stage_pair(p1, l1, p2, l2, dst);
-  };
+// The terms of a task's accumulation, kbeg <= k < kend (wave-uniform): T1_k and
+// T2_k are the 64x64 tiles 64 k columns after p1 and p2 (leading dimensions ld1,
+// ld2; T1 of the first term is at first1, ldf), and their flags lie at
+// f1 + k fs1 and f2 + k fs2.
+struct Terms {
+  int kbeg, kend;
+  const double *first1, *p1, *p2;
+  int ldf, ld1, ld2;
+  int f1, fs1, f2, fs2;
+};
+
+// acc -= sum_{kbeg <= k < kend} T1_k T2_k^T, each term once both of its tiles
+// are published.
+//
+// Terms go through two LDS buffers of 2 x 64 x 64 doubles.  A term is two
+// halves of eight 4-deep steps, whose operands are read from LDS one half
+// ahead of their MFMAs, so that with one wave on each SIMD the matrix cores
+// wait neither for LDS nor for the term's one barrier.  That barrier is in
+// the middle of the term: by then every wave has read the whole term, so its
+// buffer takes the loads of the term after next, and the next term's loads,
+// issued one term ago, have landed.
+// Which terms are published is found 64 at a time, one lane per term (a
+// scan of one flag pair at a time costs about a microsecond of memory
+// latency per term), and the next scan's loads are in flight during a half.
+// N = 997 (11N = 10967, one factorisation of each order): 16.3 -> 13.6 ms; N = 4096: 981 -> 811 ms; N = 512:
+// 3.22 -> 3.03 ms.  Past N ~ 1000 the tile reads bound it: 64 KB a term, 5.2 TB/s of L2 misses.
+__device__ __forceinline__ void pair_accumulate(v4d (&acc)[2][2], const Terms& T, const int* flags, int gen, int* err,
+                                                double* smem, int* rec, int who) {
+  const int kbeg = T.kbeg, kend = T.kend;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int* kready_x = reinterpret_cast<int*>(smem + kDagSmemDoubles) + 1;  // the scans' result by the term's parity;
+                                                                       // [2] the blocking wait's
   if (kend <= kbeg) return;
-  tile_negate(acc);
-  ready(kbeg);
-  stage(kbeg, smem);
-  __builtin_amdgcn_s_waitcnt(kWaitVm0);
-  __syncthreads();
-  for (int k = kbeg; k < kend; ++k) {
-    double* cur = smem + ((k - kbeg) & 1) * 8192;
-    double* nxt = smem + ((k - kbeg + 1) & 1) * 8192;
-    const bool more = k + 1 < kend, pre = more && k + 1 < kready;
-    pair_product(acc, pre, cur, [&] { stage(k + 1, nxt); });
-    if (more && !pre) {
-      ready(k + 1);
-      stage(k + 1, nxt);
+  int kready = kbeg;  // every term before it is known to be published
+  auto load = [&](int f) { return __hip_atomic_load(&flags[f], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+  // the first unpublished term from k on, of those that lane l's answer ok covers (term k + l)
+  auto first_not = [&](int k, bool ok) {
+    const unsigned long long no = ~__ballot(ok);
+    return k + (no ? __builtin_ctzll(no) : 64);
+  };
+  // waits for term k; takes the later ones that are already published too
+  auto ready = [&](int k) {
+    if (wave == 0) {
+      bool ok = false;
+      if (k + lane < kend) {
+        const int v1 = load(T.f1 + (k + lane) * T.fs1), v2 = load(T.f2 + (k + lane) * T.fs2);
+        ok = v1 == gen && v2 == gen;
+      }
+      int kk = first_not(k, ok);
+      if (kk == k) {
+        const int f1 = T.f1 + k * T.fs1, f2 = T.f2 + k * T.fs2;
+        if (lane == 0) {
+          wait_flag(&flags[f1], gen, err, rec, who, f1);
+          wait_flag(&flags[f2], gen, err, rec, who, f2);
+        }
+        kk = k + 1;
+      }
+      if (lane == 0) kready_x[2] = kk;
     }
-    __builtin_amdgcn_s_waitcnt(kWaitVm0);
     __syncthreads();
+    kready = __builtin_amdgcn_readfirstlane(kready_x[2]);
+    wt_seen();
+  };
+  auto term = [&](int k) {
+    const bool first = k == kbeg;
+    return TermSrc{first ? T.first1 : T.p1 + (size_t)(64 * k) * T.ld1, T.p2 + (size_t)(64 * k) * T.ld2,
+                   first ? T.ldf : T.ld1, T.ld2};
+  };
+  auto buffer = [&](int k) { return smem + ((k - kbeg) & 1) * 8192; };
+  const HalfAt at = half_at();
+  HalfOps P, Q;
+  int issued;  // terms before it are staged or on their way
+  // waits for term k, stages it and reads its first half
+  auto restart = [&](int k) {
+    ready(k);
+    const TermSrc t = term(k);
+    stage_tile(t.p1, t.ld1, buffer(k));
+    stage_tile(t.p2, t.ld2, buffer(k) + 4096);
+    issued = k + 1;
+    __builtin_amdgcn_s_waitcnt(kWaitVm0);
+    gemm_barrier();
+#pragma unroll
+    for (int u = 0; u < 8; ++u) half_read(P, at, u, 0, buffer(k));
+  };
+  // a half's products with the loads of the next term not yet issued, when it is published
+  auto half = [&](const HalfOps& use, HalfOps& next, int hnext, const double* rd, double* wr) {
+    if (issued < kready) {
+      const TermSrc t = term(issued);
+      half_product<true>(acc, use, next, at, hnext, rd, t.p1, t.ld1, t.p2, t.ld2, wr);
+      ++issued;
+    } else {
+      half_product<false>(acc, use, next, at, hnext, rd, nullptr, 0, nullptr, 0, wr);
+    }
+  };
+  tile_negate(acc);  // the terms add to the negated tile (exact: negation commutes with rounding)
+  restart(kbeg);
+  for (int k = kbeg; k < kend; ++k) {
+    // the known published terms run out: the next scan's loads
+    const bool scan = kready < kend && kready <= k + 2;
+    int v1 = gen, v2 = gen;
+    if (scan) {
+      const int kk = min(kready + lane, kend - 1);
+      v1 = load(T.f1 + kk * T.fs1);
+      v2 = load(T.f2 + kk * T.fs2);
+    }
+    // (term k+1's loads go out here only after a restart; else they are a half older)
+    if (issued == k + 1) half(P, Q, 1, buffer(k), buffer(k + 1));
+    else half_product<false>(acc, P, Q, at, 1, buffer(k), nullptr, 0, nullptr, 0, buffer(k + 1));
+    if (k + 1 == kend) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) half_mfma(acc, Q, u);
+      break;
+    }
+    __builtin_amdgcn_s_waitcnt(kWaitVm0);  // this wave's share of term k+1 has landed
+    if (scan) {
+      asm volatile("" : "+v"(v1), "+v"(v2));  // (compared here, not where they were loaded)
+      const int kk = first_not(kready, kready + lane < kend && v1 == gen && v2 == gen);
+      if (threadIdx.x == 0) kready_x[k & 1] = kk;
+    }
+    gemm_barrier();
+    if (scan) {
+      kready = __builtin_amdgcn_readfirstlane(kready_x[k & 1]);
+      wt_seen();
+    }
+    if (issued <= k + 1) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) half_mfma(acc, Q, u);
+      restart(k + 1);
+    } else {
+      half(Q, P, 0, buffer(k + 1), buffer(k));
+    }
   }
   tile_negate(acc);
+  __syncthreads();  // the staging buffers are free again
 }
 
 // out = acc Dinv^T, Dinv a column-major 64x64 tile in global memory
 __device__ __forceinline__ void tile_trsm(const v4d (&acc)[2][2], const double* __restrict__ Dg, double* smem,
                                           v4d (&out)[2][2]) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = opaque_tid(), lane = tid & 63, wave = tid >> 6;
   const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
   // Cs[kk][m] = acc(m, kk); Dinv staged, so that element (n, kk) = Dinv^T(kk, n)
   double(*Cs)[66] = reinterpret_cast<double(*)[66]>(smem);
@@ -1272,7 +1293,7 @@ __device__ __forceinline__ void tile_trsm(const v4d (&acc)[2][2], const double* 
 // tile store through LDS, so each column is written contiguously; written
 // through, every wave's stores complete at the closing barrier
 __device__ __forceinline__ void tile_store(const v4d (&out)[2][2], double* dst, int ld, double* smem) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = opaque_tid(), lane = tid & 63, wave = tid >> 6;
   const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
   double(*Cs)[66] = reinterpret_cast<double(*)[66]>(smem);
 #pragma unroll
@@ -1467,11 +1488,18 @@ __device__ __forceinline__ void dag_task(const DagArgs& g, int t, double* __rest
     return;
   }
 
-  // tickets past the factorization's: X = inv(L_S) (see potrf_lower_x)
-  if (t > nt * (nt + 1) / 2) {
-    const int s0 = g.s0, ns = nt - s0, r = t - nt * (nt + 1) / 2 - 1;
+  // A tile task: the tile (i,j) of the factor, or (past the factorization's
+  // tickets) the tile (xi,xj) of X = inv(L_S), I = s0 + xi (see potrf_lower_x)
+  const int xf = nt * nt + 2 * nt;  // X's flags, after the partial flags
+  const int s0 = g.s0, ns = nt - s0;
+  double* X = g.X;
+  const int ldx = g.ldx;
+  const bool is_x = t > nt * (nt + 1) / 2;
+  int i, j;  // the tile; of X: (xi, xj)
+  Terms T;
+  if (is_x) {
+    const int r = t - nt * (nt + 1) / 2 - 1;
     double* xdT = g.part + (size_t)2 * nt * 4096;   // X_jj^T = Dinv^T of the diagonal blocks
-    const int xf = nt * nt + 2 * nt;                 // X's flags, after the partial flags
     if (r < ns) {
       // diagonal block j: X_jj = Dinv_J into X (read by the LL^T product after
       // the launch) and its transpose (the first term's operand of block
@@ -1481,7 +1509,7 @@ __device__ __forceinline__ void dag_task(const DagArgs& g, int t, double* __rest
       __syncthreads();
       wt_seen();
       tile_load<true>(acc, g.dinv + (size_t)J * 4096, 64);
-      tile_store_direct(acc, g.X + 64 * jj + (size_t)(64 * jj) * g.ldx, g.ldx);
+      tile_store_direct(acc, X + 64 * jj + (size_t)(64 * jj) * ldx, ldx);
       tile_store_direct_t(acc, xdT + (size_t)jj * 4096, 64);
       wt_stores_done();
       __syncthreads();
@@ -1492,52 +1520,20 @@ __device__ __forceinline__ void dag_task(const DagArgs& g, int t, double* __rest
     // (I = s0 + i).  The sum is accumulated transposed, acc = -sum X_kj^T L_Ik^T,
     // from X_kj^T (kept in X's upper block (j,k); X_jj^T in xdT), so that the
     // solve with Dinv_I is tile_trsm's product: X_ij^T = acc Dinv_I^T.
-    int q = r - ns, xi = 1;
-    while (q >= xi) {
-      q -= xi;
-      ++xi;
+    j = r - ns;
+    i = 1;
+    while (j >= i) {
+      j -= i;
+      ++i;
     }
-    const int xj = q, I = s0 + xi;
-    double* X = g.X;
-    const size_t ldx = (size_t)g.ldx;
 #pragma unroll
     for (int bm = 0; bm < 2; ++bm)
 #pragma unroll
       for (int bn = 0; bn < 2; ++bn) acc[bm][bn] = (v4d){0.0, 0.0, 0.0, 0.0};
-    pair_accumulate(
-        acc, xj, xi,
-        [&](int k, const double*& p1, size_t& l1, const double*& p2, size_t& l2, int& f1, int& f2) {
-          if (k == xj) {
-            p1 = xdT + (size_t)xj * 4096;
-            l1 = 64;
-          } else {
-            p1 = X + 64 * xj + (size_t)(64 * k) * ldx;
-            l1 = ldx;
-          }
-          f1 = xf + k + ns * xj;
-          p2 = A + 64 * I + (size_t)(64 * (s0 + k)) * ld;
-          l2 = (size_t)ld;
-          f2 = I + nt * (s0 + k);
-        },
-        flags, g.gen, err, smem, rec, t);
-    if (tid == 0) wait_flag(&flags[I + nt * I], g.gen, err, rec, t, I + nt * I);
-    __syncthreads();
-    wt_seen();
-    v4d out[2][2];
-    tile_trsm(acc, g.dinv + (size_t)I * 4096, smem, out);
-    // X_ij^T into the upper block (j,i) for the later tiles of block column j;
-    // X_ij into the lower block (i,j)
-    tile_store_direct(out, X + 64 * xj + (size_t)(64 * xi) * ldx, ldx);
-    tile_store_direct_t(out, X + 64 * xi + (size_t)(64 * xj) * ldx, ldx);
-    wt_stores_done();
-    __syncthreads();
-    if (tid == 0) wt_publish(&flags[xf + xi + ns * xj], g.gen);
-    return;
-  }
-
-  // the tile of ticket t (see above)
-  int i, j;
-  {
+    const int I = s0 + i;
+    T = Terms{j, i, xdT + (size_t)j * 4096, X + 64 * j, A + 64 * I + (size_t)(64 * s0) * ld,
+              64, ldx, ld, xf + ns * j, 1, I + nt * s0, nt};
+  } else {
     auto esize = [nt](int c) { return c < nt ? min(kEarly, nt - c) : 0; };  // early tiles of column c
     int r = t - 1, c0 = 0;
     for (; c0 < kAhead && c0 < nt; ++c0) {
@@ -1563,25 +1559,37 @@ __device__ __forceinline__ void dag_task(const DagArgs& g, int t, double* __rest
         r -= o;
       }
     }
-  }
-  tile_load(acc, A + 64 * i + (size_t)(64 * j) * ld, ld);
-  if (i == j || i == j + 1) {
+    tile_load(acc, A + 64 * i + (size_t)(64 * j) * ld, ld);
     // partial sums for the walker: (j,j) without its last term, (j+1,j) complete
-    tile_accumulate(acc, A, ld, nt, i, j, i == j ? max(j - 1, 0) : j, flags, g.gen, err, smem, rec, t);
+    T = Terms{0, i == j ? max(j - 1, 0) : j, A + 64 * i, A + 64 * i, A + 64 * j, ld, ld, ld, i, nt, j, nt};
+  }
+  pair_accumulate(acc, T, flags, g.gen, err, smem, rec, t);
+  if (!is_x && i - j <= 1) {
     tile_store_direct(acc, g.part + (size_t)(2 * j + (i - j)) * 4096, 64);
     wt_stores_done();
     __syncthreads();
     if (tid == 0) wt_publish(&pflags[2 * j + (i - j)], g.gen);
     return;
   }
-  tile_accumulate(acc, A, ld, nt, i, j, j, flags, g.gen, err, smem, rec, t);
-  if (tid == 0) wait_flag(&flags[j + nt * j], g.gen, err, rec, t, j + nt * j);
+  // the solve with the walker's diagonal inverse: of column j, or of X's row
+  const int D = is_x ? s0 + i : j;
+  if (tid == 0) wait_flag(&flags[D + nt * D], g.gen, err, rec, t, D + nt * D);
   __syncthreads();
   wt_seen();
   v4d out[2][2];
-  tile_trsm(acc, g.dinv + (size_t)j * 4096, smem, out);
-  tile_store(out, A + 64 * i + (size_t)(64 * j) * ld, ld, smem);
-  if (tid == 0) wt_publish(&flags[i + nt * j], g.gen);
+  tile_trsm(acc, g.dinv + (size_t)D * 4096, smem, out);
+  if (is_x) {
+    // X_ij^T into the upper block (j,i) for the later tiles of block column j;
+    // X_ij into the lower block (i,j)
+    tile_store_direct(out, X + 64 * j + (size_t)(64 * i) * ldx, ldx);
+    tile_store_direct_t(out, X + 64 * i + (size_t)(64 * j) * ldx, ldx);
+    wt_stores_done();
+    __syncthreads();
+    if (tid == 0) wt_publish(&flags[xf + i + ns * j], g.gen);
+  } else {
+    tile_store(out, A + 64 * i + (size_t)(64 * j) * ld, ld, smem);
+    if (tid == 0) wt_publish(&flags[i + nt * j], g.gen);
+  }
 }
 
 // The launch is persistent: as many workgroups as the GPU holds at once
@@ -1595,8 +1603,11 @@ __device__ __forceinline__ void dag_task(const DagArgs& g, int t, double* __rest
 // left to start is full of waiting ones, the lowest untaken ticket never
 // starts.)
 __global__ __launch_bounds__(256) void potrf_dag_kernel(DagArgs g) {
-  __shared__ __attribute__((aligned(16))) double smem[kDagSmemDoubles];
-  __shared__ int t_s;
+  // one LDS variable: with several, the compiler's record of which pointers
+  // are distinct is lost, and LDS reads wait for every load into LDS before
+  // them (half_product)
+  __shared__ __attribute__((aligned(16))) double smem[kDagSmemDoubles + 2];
+  int& t_s = *reinterpret_cast<int*>(smem + kDagSmemDoubles);  // then the three words of pair_accumulate
   const int ns = g.s0 >= 0 ? g.nt - g.s0 : 0;
   const int total = g.nt * (g.nt + 1) / 2 + ns * (ns + 1) / 2;  // the last ticket
   for (;;) {
@@ -1609,7 +1620,7 @@ __global__ __launch_bounds__(256) void potrf_dag_kernel(DagArgs g) {
         __hip_atomic_store(&g.sync[0], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     __syncthreads();
-    const int t = t_s;
+    const int t = __builtin_amdgcn_readfirstlane(t_s);
     __syncthreads();
     if (t > total) break;
     dag_task(g, t, smem);

@@ -144,8 +144,8 @@ __global__ __launch_bounds__(64) void ewald_pair_kernel(EwaldParams p, const dou
                                                         const double* __restrict__ radii,
                                                         const double* __restrict__ kw, double* __restrict__ G,
                                                         int* __restrict__ n_overlap) {
-  // the N(N-1)/2 pairs alpha < beta packed 64 to a wave in row-major order;
-  // the last wave's spare lanes repeat the last pair
+  // the pairs alpha < beta packed 64 to a wave in row-major order; the last
+  // wave's spare lanes repeat the last pair
   int al, be;
   const bool active = pair_of_lane((long long)blockIdx.x * 64 + threadIdx.x, p.N, al, be);
   const int bq = be;
@@ -225,6 +225,132 @@ __global__ __launch_bounds__(64) void ewald_pair_kernel(EwaldParams p, const dou
   scatter_pair(G, p.ld, p.offT, p.offR, p.offQ, al, be, o, p.inv_pimu);
 }
 
+// The same sum with each pair split over kSplitWaves waves of a workgroup and
+// L lanes of each, from pair `first` on: the images and the rows of wave
+// vectors are dealt out, the partial blocks added through LDS in a fixed
+// order; 64 / L pairs a workgroup, and a workgroup a CU (400 VGPRs, one wave
+// on each SIMD).  One lane's serial image sum bounds the kernel above while
+// its waves are fewer than the chip's 1024 SIMDs, whatever N is: at N = 16 a
+// whole assembly took 187 us with half-widths 2 and 472 us with 3, and takes 37
+// and 53 us with the split (this kernel 21 us of the 37).
+constexpr int kSplitWaves = 4;
+constexpr int kPairOut = 60;  // doubles of a PairOut
+static_assert(sizeof(PairOut) == kPairOut * sizeof(double), "PairOut is an array of doubles");
+
+template <int L>
+__global__ __launch_bounds__(64 * kSplitWaves) void ewald_pair_split_kernel(EwaldParams p,
+                                                                            const double* __restrict__ pos,
+                                                                            const double* __restrict__ radii,
+                                                                            const double* __restrict__ kw,
+                                                                            double* __restrict__ G,
+                                                                            int* __restrict__ n_overlap,
+                                                                            long long first) {
+  constexpr int P = 64 / L, S = kSplitWaves, kRound = 15;
+  __shared__ double part[S][kRound][P];
+  __shared__ double fin[kPairOut][P];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int pr = lane / L, sub = lane % L;
+  int al, be;
+  const bool active = pair_of_lane(first + (long long)blockIdx.x * P + pr, p.N, al, be);
+  const double ai = radii[al], aj = radii[be];
+  const double ai2 = ai * ai, aj2 = aj * aj;
+  double Rx = pos[3 * al] - pos[3 * be], Ry = pos[3 * al + 1] - pos[3 * be + 1], Rz = pos[3 * al + 2] - pos[3 * be + 2];
+  const double dmin = skew_correction(p, Rx, Ry, Rz);
+
+  PairOut o;
+  pairout_zero(o);
+  Radial s;
+  const int sr = 2 * p.NR + 1, nimg = sr * sr * sr;
+  for (int t = wave * L + sub; t < nimg; t += S * L) {  // nz fastest, as nested loops over nx, ny, nz
+    const int nx = t / (sr * sr) - p.NR, ny = (t / sr) % sr - p.NR, nz = t % sr - p.NR;
+    const double x = Rx + (p.LR[0] * nx + p.LR[3] * ny + p.LR[6] * nz);
+    const double y = Ry + (p.LR[1] * nx + p.LR[4] * ny + p.LR[7] * nz);
+    const double z = Rz + (p.LR[2] * nx + p.LR[5] * ny + p.LR[8] * nz);
+    radial_ewald(sqrt(x * x + y * y + z * z), p.lam, s);
+    radial_block(x, y, z, s, ai2, aj2, p.phix, true, 1.0, o);
+  }
+  // k space over the positive half of the cube, doubled (as above), by whole
+  // rows (n1, n2), dealt out like the images (with L = 1 a wave's row is the
+  // same for all lanes, and its weights are wave-uniform scalar loads)
+  {
+    double X[3];
+    for (int i = 0; i < 3; ++i) X[i] = p.LI[i] * Rx + p.LI[i + 3] * Ry + p.LI[i + 6] * Rz;
+    double wc, ws;
+    sincos(2.0 * kPi * X[2], &ws, &wc);
+    const int NI = p.NI, side = 2 * NI + 1;
+    // rows in order of (n1, n2) from (0, 0), whose n3 starts at 1
+    const int rows = (side * side + 1) / 2, row0 = side * side / 2;
+    for (int r = L > 1 ? wave * L + sub : wave; r < rows; r += S * L) {
+      const int n1 = (row0 + r) / side - NI, n2 = (row0 + r) % side - NI, n3lo = r == 0 ? 1 : -NI;
+      double zc, zs;
+      sincos(2.0 * kPi * (n1 * X[0] + n2 * X[1] + n3lo * X[2]), &zs, &zc);
+      zc *= 2.0;
+      zs *= 2.0;
+      const double* kwrow = kw + (size_t)((row0 + r) * side + NI) * kKW;  // n3 = 0
+      for (int n3 = n3lo; n3 <= NI; ++n3) {
+        kspace_accumulate(kwrow + (ptrdiff_t)n3 * kKW, zc, zs, ai2, aj2, p.phix, o);
+        const double tc = zc * wc - zs * ws;
+        zs = zc * ws + zs * wc;
+        zc = tc;
+      }
+    }
+  }
+  if (wave == 0 && sub == 0 && active && p.correction_method != 0 && dmin <= ai + aj) {
+    // per_GRPY_YZD.f90:98-116: 1 Yamakawa, 2 regularised
+    if (p.correction_method == 1)
+      overlap_yamakawa_correction(Rx, Ry, Rz, ai, aj, o);
+    else
+      overlap_regular_correction(Rx, Ry, Rz, ai, aj, o);
+    atomicAdd(n_overlap, 1);
+  }
+  // the sum over a pair's lanes, then over the waves, kRound of the 60 numbers at a time
+  double v[kPairOut];
+  __builtin_memcpy(v, &o, sizeof o);
+#pragma unroll
+  for (int q = 0; q < kPairOut; ++q)
+#pragma unroll
+    for (int off = L / 2; off > 0; off >>= 1) v[q] += __shfl_xor(v[q], off, 64);
+#pragma unroll
+  for (int r = 0; r < kPairOut / kRound; ++r) {
+    if (sub == 0)
+#pragma unroll
+      for (int q = 0; q < kRound; ++q) part[wave][q][pr] = v[r * kRound + q];
+    __syncthreads();
+    for (int e = threadIdx.x; e < kRound * P; e += 64 * S) {
+      double sum = 0.0;
+#pragma unroll
+      for (int w = 0; w < S; ++w) sum += part[w][e / P][e % P];
+      fin[r * kRound + e / P][e % P] = sum;
+    }
+    __syncthreads();
+  }
+  // scatter (per_GRPY_YZD.f90:122-188), scaled by 1/(pi mu_f): a pair a lane
+  if (threadIdx.x >= P) return;
+  const bool mine = pair_of_lane(first + (long long)blockIdx.x * P + threadIdx.x, p.N, al, be);
+  if (!mine) return;
+#pragma unroll
+  for (int q = 0; q < kPairOut; ++q) v[q] = fin[q][threadIdx.x];
+  __builtin_memcpy(&o, v, sizeof o);
+  scatter_pair(G, p.ld, p.offT, p.offR, p.offQ, al, be, o, p.inv_pimu);
+}
+
+// Lanes of a wave that share a pair in the split kernel, for `np` pairs; 0: a
+// lane a pair in the kernel above.  A split pays while its workgroups make one
+// round over the 256 CUs (two without sharing lanes: a quarter of the serial
+// sum each).  Assembly in us, lanes 16 / 4 / 1 / no split, half-widths 2:
+//   N = 32 (496 pairs)      38 /  51 /  80 / 188
+//   N = 64 (2016)           58 /  52 /  81 / 189
+//   N = 100 (4950)         117 /  86 /  85 / 191
+//   N = 240 (28680)        557 / 294 / 179 / 230
+//   N = 280 (39060)        741 / 369 / 255 / 254
+// and in the same order with half-widths 3 and with 4 and 6.
+static int pair_split(long long np) {
+  if (np <= 256 * 4) return 16;
+  if (np <= 256 * 16) return 4;
+  if (np <= 2 * 256 * 64) return 1;
+  return 0;
+}
+
 int ewald_assemble(const EwaldParams& p, const double* d_pos, const double* d_radii, double* d_kw, double* G,
                    int* d_overlap, hipStream_t s, bool profiled) {
   const int side = 2 * p.NI + 1, total = side * side * side;
@@ -236,11 +362,25 @@ int ewald_assemble(const EwaldParams& p, const double* d_pos, const double* d_ra
   prof_end(pe, s);
   if (p.N > 1) {
     const long long np = (long long)p.N * (p.N - 1) / 2;
-    dim3 grid((unsigned)((np + 63) / 64));
     const double pairs = 0.5 * (double)p.N * (p.N - 1);
     hipEvent_t pp =
         profiled ? prof_begin(kProfEwaldPair, pairs * (1000.0 * nr3 + 250.0 * nk), pairs * 242.0 * 8.0, s) : nullptr;
-    hipLaunchKernelGGL(ewald_pair_kernel, grid, dim3(64), 0, s, p, d_pos, d_radii, (const double*)d_kw, G, d_overlap);
+    // whole rounds of waves (one a SIMD, 64 pairs each) go a lane a pair; a
+    // last round that would be less than half full is split instead (N = 400:
+    // 65536 + 14264 pairs)
+    const long long round = 1024 * 64, whole = np / round * round;
+    const int split = pair_split(np - whole);
+    const long long plain = split ? whole : np;
+    if (plain > 0)
+      hipLaunchKernelGGL(ewald_pair_kernel, dim3((unsigned)((plain + 63) / 64)), dim3(64), 0, s, p, d_pos, d_radii,
+                         (const double*)d_kw, G, d_overlap);
+    if (plain < np) {
+      const int per = 64 / split;
+      auto kern = split == 16 ? ewald_pair_split_kernel<16>
+                              : split == 4 ? ewald_pair_split_kernel<4> : ewald_pair_split_kernel<1>;
+      hipLaunchKernelGGL(kern, dim3((unsigned)((np - plain + per - 1) / per)), dim3(64 * kSplitWaves), 0, s, p, d_pos,
+                         d_radii, (const double*)d_kw, G, d_overlap, plain);
+    }
     prof_end(pp, s);
   }
   RSD_HIP(hipGetLastError());

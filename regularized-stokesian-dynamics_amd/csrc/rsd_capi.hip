@@ -1092,8 +1092,10 @@ struct rsd_gnn {
 static bool precond_learned(int p) { return p == RSD_PRECOND_LEARNED || p == RSD_PRECOND_MIXED_LEARNED; }
 static bool precond_mixed(int p) { return p == RSD_PRECOND_MIXED || p == RSD_PRECOND_MIXED_LEARNED; }
 
-// The FP32 copy of M: columns padded to 16 bytes for the vector loads
+// The FP32 copies: blocks, self blocks, then M from a 16-byte boundary with its
+// columns padded to 16 bytes, for the vector loads
 static int iter_ld32(int n11) { return (n11 + 3) & ~3; }
+static size_t iter_m32(int N, int cap) { return ((size_t)N * (cap + 1) * 121 + 3) & ~(size_t)3; }
 
 // Buffers of the iterative route (its Krylov space, the block-sparse
 // lubrication, FP32 copies for the mixed preconditioners, the learned
@@ -1107,7 +1109,7 @@ static int iter_buffers(rsd_ctx* c, int precond, int nz) {
   RSD_TRY(c->bit.alloc(2 * (size_t)n11));
   RSD_TRY(c->wit.alloc(2 * (size_t)n11));
   if (!c->bsr_ix) RSD_HIP(hipMalloc(&c->bsr_ix, ((size_t)N * (cap + 1) + 1) * sizeof(int)));
-  const size_t n32 = (size_t)N * cap * 121 + (size_t)N * 121 + (size_t)iter_ld32(n11) * n11;
+  const size_t n32 = iter_m32(N, cap) + (size_t)iter_ld32(n11) * n11;
   if (precond_mixed(precond) && c->bsr32_cap < n32) {
     if (c->bsr32) RSD_HIP(hipFree(c->bsr32));
     c->bsr32 = nullptr;
@@ -1164,7 +1166,7 @@ static GmresSetup iter_setup(rsd_ctx* c, int precond, const LubBsr<double>* L, L
   const int N = c->N, cap = rsd_ctx::kBsrCap, n11 = c->n11;
   const bool mixed = precond_mixed(precond);
   float* self32 = mixed ? c->bsr32 + (size_t)N * cap * 121 : nullptr;
-  float* M32 = mixed ? self32 + (size_t)N * 121 : nullptr;
+  float* M32 = mixed ? c->bsr32 + iter_m32(N, cap) : nullptr;
   *L32 = LubBsr<float>{N, cap, c->bsr_ix, c->bsr_ix + N, mixed ? c->bsr32 : nullptr, self32};
   GmresSetup gs{L, c->G.p, c->n11p, L32, M32, iter_ld32(n11), precond, c->it_inner, L};
   gs.graphs = c->it_graphs;
@@ -1600,12 +1602,12 @@ extern "C" int rsd_ctx_step(rsd_ctx* c, double dt, double t, double yeta_mu[5]) 
         if (!res.converged) return 1;
       }
       // U = (M x)_P
-      RSD_TRY(dense_gemv<double>(c->G.p, n11p, n11, c->xit.p, c->wit.p, c->iw.part, s));
+      RSD_TRY(dense_gemv<double>(c->G.p, n11p, n11, c->xit.p, c->wit.p, s));
       RSD_HIP(hipMemcpyAsync(x0, c->wit.p, n6 * sizeof(double), hipMemcpyDeviceToDevice, s));
       if (sub == 0) RSD_HIP(hipEventRecord(c->ev[4], s));
       if (sub == nt - 1) {
         const double* xs = c->xit.p + (size_t)(nsolve - 1) * n11;
-        RSD_TRY(dense_gemv<double>(c->G.p, n11p, n11, xs, c->wit.p, c->iw.part, s));
+        RSD_TRY(dense_gemv<double>(c->G.p, n11p, n11, xs, c->wit.p, s));
         RSD_TRY(bsr_apply<double>(L, c->wit.p, c->wit.p + n11, false, s));
         RSD_TRY(vector_sum(xs + n6, c->wit.p + n11 + n6, c->shyd.p, n5, s));
       }
@@ -1880,7 +1882,7 @@ extern "C" int rsd_ctx_gnn_loss(rsd_ctx* c, rsd_gnn* g, int nz, unsigned long lo
   const LubBsr<double> L = iter_bsr(c);
   RSD_TRY(gnn_forward(c->gw, g->m.p, L, c->iw.corr, s));
   RSD_TRY(gnn_loss_grad(c->gw, g->m.p, L, c->G.p, c->n11p, c->iw.dinv, c->iw.corr, nz, seed, 0, grad != nullptr,
-                        false, c->iw.part, loss, s));
+                        false, loss, s));
   if (grad) RSD_HIP(hipMemcpy(grad, c->gw.grad, kGnnParams * sizeof(float), hipMemcpyDeviceToHost));
   if (z) RSD_HIP(hipMemcpy(z, c->gw.zv, (size_t)nz * c->n11 * sizeof(double), hipMemcpyDeviceToHost));
   return RSD_OK;
@@ -1896,7 +1898,7 @@ extern "C" int rsd_ctx_gnn_train(rsd_ctx* c, rsd_gnn* g, int iters, int nz, floa
     double loss = 0.0;
     RSD_TRY(gnn_forward(c->gw, g->m.p, L, c->iw.corr, s));
     RSD_TRY(gnn_loss_grad(c->gw, g->m.p, L, c->G.p, c->n11p, c->iw.dinv, c->iw.corr, nz, seed,
-                          (unsigned long long)it + 1, true, true, c->iw.part, &loss, s));
+                          (unsigned long long)it + 1, true, true, &loss, s));
     RSD_TRY(gnn_adam(g->m, c->gw.grad, lr, s));
     if (losses) losses[it] = loss;
   }

@@ -97,10 +97,10 @@ int gnn_prepare(GnnWork& w, const LubBsr<double>& L, const double* M, int ld, co
 int gnn_forward(GnnWork& w, const float* params, const LubBsr<double>& L, double* corr, hipStream_t s);
 // The loss for nz Gaussian vectors drawn from (seed, draw) and, when grad,
 // its gradient with respect to the parameters into w.grad (log_loss: of
-// log(loss)).  Needs gnn_forward's activations; part: dense_gemv's scratch.
+// log(loss)).  Needs gnn_forward's activations.
 int gnn_loss_grad(GnnWork& w, const float* params, const LubBsr<double>& L, const double* M, int ld,
                   const double* dinv, const double* corr, int nz, unsigned long long seed, unsigned long long draw,
-                  bool grad, bool log_loss, double* part, double* loss, hipStream_t s);
+                  bool grad, bool log_loss, double* loss, hipStream_t s);
 // One Adam step of the model with w.grad.
 int gnn_adam(GnnModel& g, const float* grad, float lr, hipStream_t s);
 

@@ -606,7 +606,7 @@ int gnn_forward(GnnWork& w, const float* params, const LubBsr<double>& L, double
 
 int gnn_loss_grad(GnnWork& w, const float* params, const LubBsr<double>& L, const double* M, int ld,
                   const double* dinv, const double* corr, int nz, unsigned long long seed, unsigned long long draw,
-                  bool grad, bool log_loss, double* part, double* loss, hipStream_t s) {
+                  bool grad, bool log_loss, double* loss, hipStream_t s) {
   const int N = L.N, n = 11 * N, n6 = 6 * N;
   if (nz < 1 || nz > w.nz) {
     set_error("gnn_loss_grad: nz outside the reserved buffers");
@@ -615,7 +615,7 @@ int gnn_loss_grad(GnnWork& w, const float* params, const LubBsr<double>& L, cons
   const dim3 blk(256), grd((n + 255) / 256);
   double* y = w.wv;
   double* r = w.wv + n;
-  double* kw = w.wv + 2 * (size_t)n;  // apply_k's scratch (2n)
+  double* kw = w.wv + 2 * (size_t)n;  // apply_k's scratch
   double* t = w.wv + 4 * (size_t)n;
   hipLaunchKernelGGL(zero2_kernel, dim3(1), dim3(64), 0, s, w.red);
   for (int z = 0; z < nz; ++z) {
@@ -623,7 +623,7 @@ int gnn_loss_grad(GnnWork& w, const float* params, const LubBsr<double>& L, cons
     RSD_TRY(launch_brown_normal(n, seed, draw * 4096ull + (unsigned long long)z, Zz, s));
     // r = K P z - z
     RSD_TRY(block_apply<double>(N, dinv, corr, &L, Zz, y, s));
-    RSD_TRY(apply_k<double>(L, M, ld, y, r, kw, part, s));
+    RSD_TRY(apply_k<double>(L, M, ld, y, r, kw, s));
     hipLaunchKernelGGL(axpby_kernel, grd, blk, 0, s, n, 1.0, (const double*)r, -1.0, (const double*)Zz, r);
     hipLaunchKernelGGL(sumsq2_kernel, dim3(1), blk, 0, s, n, (const double*)r, (const double*)Zz, w.red);
     if (!grad) continue;
@@ -633,7 +633,7 @@ int gnn_loss_grad(GnnWork& w, const float* params, const LubBsr<double>& L, cons
     RSD_TRY(bsr_apply<double>(L, t, y, false, s));
     hipLaunchKernelGGL(keep_rows_kernel, grd, blk, 0, s, n, n6, (const double*)r, kw, 0);
     hipLaunchKernelGGL(axpby_kernel, grd, blk, 0, s, n, 1.0, (const double*)y, 1.0, (const double*)kw, y);
-    RSD_TRY(dense_gemv<double>(M, ld, n, y, Gz, part, s));
+    RSD_TRY(dense_gemv<double>(M, ld, n, y, Gz, s));
     hipLaunchKernelGGL(axpby_kernel, grd, blk, 0, s, n, 1.0, (const double*)Gz, 1.0, (const double*)t, Gz);
   }
   RSD_HIP(hipGetLastError());

@@ -39,14 +39,15 @@ struct IterWork {
   double* V = nullptr;       // (m+1) Krylov vectors
   double* Z = nullptr;       // m preconditioned vectors (flexible GMRES)
   double* w = nullptr;       // work: 4 vectors
-  double* part = nullptr;    // split-K partial sums
-  double* h = nullptr;       // device Hessenberg column + norm
-  double* hh = nullptr;      // pinned host copy
+  double* h = nullptr;       // norms, and the triangular system's solution (and, after it, the vectors below)
+  double* hcol = nullptr;    // device Hessenberg column, then the norm's partial sums
+  double* hh = nullptr;      // pinned host copy of hcol
+  // partial sums of the two Gram-Schmidt passes, of squared norms; the first
+  // pass's coefficients; reciprocal norms of the FP32 Krylov vectors; ones
+  double *part1 = nullptr, *part2 = nullptr, *partn = nullptr, *h1 = nullptr, *inv = nullptr, *ones = nullptr;
   float* V32 = nullptr;      // FP32 inner solver's Krylov and work vectors
   float* w32 = nullptr;
-  float* part32 = nullptr;
   float* h32 = nullptr;
-  float* hh32 = nullptr;
   double* dinv = nullptr;    // block-Jacobi inverses, 121 per particle
   float* dinv32 = nullptr;
   double* corr = nullptr;    // learned correction blocks (self + neighbour slots), 121 each
@@ -64,12 +65,12 @@ struct IterWork {
 int iter_reserve(IterWork& w, int n11, int m, int N, int bsr_cap);
 void iter_release(IterWork& w);
 
-// y = M x for a dense column-major M (n x n, leading ld), split over K.
+// y = M x for a dense symmetric M (n x n, both triangles, leading ld; x and y distinct).
 template <typename T>
-int dense_gemv(const T* M, int ld, int n, const T* x, T* y, T* part, hipStream_t s);
-// y = x_P + (R_lub (M x))_P rows, y_Q = (M x)_Q: the operator K.
+int dense_gemv(const T* M, int ld, int n, const T* x, T* y, hipStream_t s);
+// y = x_P + (R_lub (M x))_P rows, y_Q = (M x)_Q: the operator K (wbuf: M x).
 template <typename T>
-int apply_k(const LubBsr<T>& L, const T* M, int ld, const T* x, T* y, T* wbuf, T* part, hipStream_t s);
+int apply_k(const LubBsr<T>& L, const T* M, int ld, const T* x, T* y, T* wbuf, hipStream_t s);
 // lw = R_lub w (all 11N rows)
 template <typename T>
 int bsr_apply(const LubBsr<T>& L, const T* w, T* lw, bool p_rows_only, hipStream_t s);
@@ -112,7 +113,6 @@ int gmres_solve(IterWork& w, const GmresSetup& g, const double* b, double* x, do
 
 // field-major <-> FP32 copies
 int to_f32(const double* x, float* y, size_t n, hipStream_t s);
-int to_f64(const float* x, double* y, size_t n, hipStream_t s);
 int matrix_to_f32(const double* A, int lda, float* B, int ldb, int m, int n, hipStream_t s);
 
 }  // namespace rsd

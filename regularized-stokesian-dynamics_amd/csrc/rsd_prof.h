@@ -14,8 +14,8 @@ enum ProfFamily : int {
   kProfLub = 5,       // lub_kernel
   kProfGemv = 6,      // gemv kernels
   kProfPcg = 7,       // pcg_kernel (one conjugate-gradient solve per record)
-  kProfGemvSplit64 = 8,  // gemv_split_kernel<double> + its sum (the iterative route's M products, FP64)
-  kProfGemvSplit32 = 9,  // gemv_split_kernel<float> + its sum (the mixed preconditioner's, FP32)
+  kProfGemvSplit64 = 8,  // sym_gemv_kernel<double> (the iterative route's M products, FP64)
+  kProfGemvSplit32 = 9,  // sym_gemv_kernel<float> (the mixed preconditioner's, FP32)
   kProfInnerGraph = 10,  // one replay of the captured FP32 inner GMRES (the mixed preconditioner)
   kProfFamilies = 11
 };

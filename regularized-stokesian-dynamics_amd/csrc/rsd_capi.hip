@@ -255,17 +255,199 @@ struct DBuf {
   }
 };
 
-// host <-> device copies of a column-major sub-block
+// Device memory of the host-array entry points: each thread keeps one block and
+// hands it out from the front while a call runs (a hipMalloc and a hipFree a
+// matrix took longer than the algebra at N = 100).  What a call needs beyond
+// the block comes from hipMalloc and goes back at its end; the block then grows
+// to what the call used, up to kArenaMax, at the start of the thread's next
+// call.  The entry points run on the null stream and end with a wait for it, so
+// a call finds the block free.
+constexpr size_t kArenaMax = 512u << 20;
+struct DeviceArena {
+  int dev = -1, live = 0;
+  char* base = nullptr;
+  size_t cap = 0, used = 0, total = 0;  // the block's size, its part in use, all that the last call asked for
+  std::vector<void*> extra;
+  ~DeviceArena() { drop(); }
+  void drop() {
+    if (base) (void)hipFree(base);
+    base = nullptr;
+    cap = 0;
+  }
+  int get(size_t bytes, void** p) {
+    bytes = (std::max<size_t>(bytes, 1) + 255) & ~(size_t)255;
+    if (live == 0) {
+      int d = 0;
+      RSD_HIP(hipGetDevice(&d));
+      const size_t want = std::min(total, kArenaMax);
+      if (d != dev || want > cap) {
+        drop();
+        dev = d;
+        if (want > 0) {
+          void* q = nullptr;
+          if (hipMalloc(&q, want) == hipSuccess) {
+            base = static_cast<char*>(q);
+            cap = want;
+          } else {
+            (void)hipGetLastError();  // the call's own allocations report it
+          }
+        }
+      }
+      used = 0;
+      total = 0;
+    }
+    if (used + bytes <= cap) {
+      *p = base + used;
+      used += bytes;
+    } else {
+      void* q = nullptr;
+      RSD_HIP(hipMalloc(&q, bytes));
+      extra.push_back(q);
+      *p = q;
+    }
+    total += bytes;
+    ++live;
+    return RSD_OK;
+  }
+  void put() {
+    if (--live > 0) return;
+    for (void* q : extra) (void)hipFree(q);
+    extra.clear();
+  }
+};
+static DeviceArena& device_arena() {
+  static thread_local DeviceArena a;
+  return a;
+}
+struct ArenaBuf {
+  double* p = nullptr;
+  ArenaBuf() = default;
+  ArenaBuf(const ArenaBuf&) = delete;
+  ArenaBuf& operator=(const ArenaBuf&) = delete;
+  ~ArenaBuf() {
+    if (p) device_arena().put();
+  }
+  int alloc(size_t count) {  // once
+    void* q = nullptr;
+    RSD_TRY(device_arena().get(count * sizeof(double), &q));
+    p = static_cast<double*>(q);
+    return RSD_OK;
+  }
+};
+
+// Copies between a caller's host matrix and the device, through two pinned
+// halves a thread: the host fills (or empties) one while the other is on its
+// way.  A copy straight from pageable memory pins and unpins the caller's pages
+// on every call: 2.9 ms for a matrix of 2.9 MB.  rsd_stepper_nogmres at N = 100
+// took 37 ms for 1.5 ms of kernels and takes 2.1; rsd_matrev at n = 6600 185 ms,
+// now 56.
+constexpr size_t kStageDoubles = (4u << 20) / sizeof(double);  // a half
+struct HostStage {
+  int dev = -1;
+  double* half[2] = {};
+  hipEvent_t ev[2] = {};
+  bool busy[2] = {};
+  int next = 0;
+  ~HostStage() { drop(); }
+  void drop() {
+    for (int k = 0; k < 2; ++k) {
+      if (busy[k]) (void)hipEventSynchronize(ev[k]);
+      if (ev[k]) (void)hipEventDestroy(ev[k]);
+      if (half[k]) (void)hipHostFree(half[k]);
+      half[k] = nullptr;
+      ev[k] = nullptr;
+      busy[k] = false;
+    }
+    dev = -1;
+  }
+  int ready() {
+    int d = 0;
+    RSD_HIP(hipGetDevice(&d));
+    if (d == dev) return RSD_OK;
+    drop();
+    for (int k = 0; k < 2; ++k) {
+      RSD_HIP(hipHostMalloc(reinterpret_cast<void**>(&half[k]), kStageDoubles * sizeof(double)));
+      RSD_HIP(hipEventCreateWithFlags(&ev[k], hipEventDisableTiming));
+    }
+    dev = d;
+    return RSD_OK;
+  }
+  int wait(int k) {
+    if (busy[k]) RSD_HIP(hipEventSynchronize(ev[k]));
+    busy[k] = false;
+    return RSD_OK;
+  }
+  int sent(int k, hipStream_t s) {
+    RSD_HIP(hipEventRecord(ev[k], s));
+    busy[k] = true;
+    return RSD_OK;
+  }
+};
+static HostStage& host_stage() {
+  static thread_local HostStage st;
+  return st;
+}
+static void copy_columns(double* dst, int ldd, const double* src, int lds, int m, int n) {
+  if (ldd == m && lds == m) {
+    memcpy(dst, src, (size_t)m * n * sizeof(double));
+    return;
+  }
+  for (int c = 0; c < n; ++c) memcpy(dst + (size_t)c * ldd, src + (size_t)c * lds, (size_t)m * sizeof(double));
+}
+static hipError_t copy_2d(void* dst, int ldd, const void* src, int lds, int m, int n, hipMemcpyKind kind,
+                          hipStream_t s) {
+  const size_t e = sizeof(double);
+  if (ldd == m && lds == m) return hipMemcpyAsync(dst, src, (size_t)m * n * e, kind, s);
+  return hipMemcpy2DAsync(dst, ldd * e, src, lds * e, m * e, n, kind, s);
+}
+
+// host <-> device copies of a column-major sub-block; the host side is done
+// when they return
 static int d2h_block(const double* dsrc, int ldd, double* h, int ldh, int m, int n, hipStream_t s) {
   if (m <= 0 || n <= 0) return RSD_OK;
-  RSD_HIP(hipMemcpy2DAsync(h, (size_t)ldh * sizeof(double), dsrc, (size_t)ldd * sizeof(double), (size_t)m * sizeof(double),
-                           n, hipMemcpyDeviceToHost, s));
-  return RSD_OK;
+  if ((size_t)m > kStageDoubles) {
+    RSD_HIP(copy_2d(h, ldh, dsrc, ldd, m, n, hipMemcpyDeviceToHost, s));
+    RSD_HIP(hipStreamSynchronize(s));
+    return RSD_OK;
+  }
+  HostStage& st = host_stage();
+  RSD_TRY(st.ready());
+  const int step = (int)std::min<size_t>(n, kStageDoubles / m);
+  int done = -1, done_k = 0;  // the chunk on its way: its first column and half
+  auto out = [&]() -> int {
+    RSD_TRY(st.wait(done_k));
+    copy_columns(h + (size_t)done * ldh, ldh, st.half[done_k], m, m, std::min(step, n - done));
+    return RSD_OK;
+  };
+  for (int c = 0; c < n; c += step) {
+    const int k = st.next;
+    st.next ^= 1;
+    RSD_TRY(st.wait(k));
+    RSD_HIP(copy_2d(st.half[k], m, dsrc + (size_t)c * ldd, ldd, m, std::min(step, n - c), hipMemcpyDeviceToHost, s));
+    RSD_TRY(st.sent(k, s));
+    if (done >= 0) RSD_TRY(out());
+    done = c;
+    done_k = k;
+  }
+  return out();
 }
 static int h2d_block(const double* h, int ldh, double* ddst, int ldd, int m, int n, hipStream_t s) {
   if (m <= 0 || n <= 0) return RSD_OK;
-  RSD_HIP(hipMemcpy2DAsync(ddst, (size_t)ldd * sizeof(double), h, (size_t)ldh * sizeof(double), (size_t)m * sizeof(double),
-                           n, hipMemcpyHostToDevice, s));
+  if ((size_t)m > kStageDoubles) {
+    RSD_HIP(copy_2d(ddst, ldd, h, ldh, m, n, hipMemcpyHostToDevice, s));
+    return RSD_OK;
+  }
+  HostStage& st = host_stage();
+  RSD_TRY(st.ready());
+  const int step = (int)std::min<size_t>(n, kStageDoubles / m);
+  for (int c = 0; c < n; c += step) {
+    const int k = st.next, w = std::min(step, n - c);
+    st.next ^= 1;
+    RSD_TRY(st.wait(k));
+    copy_columns(st.half[k], m, h + (size_t)c * ldh, ldh, m, w);
+    RSD_HIP(copy_2d(ddst + (size_t)c * ldd, ldd, st.half[k], m, m, w, hipMemcpyHostToDevice, s));
+    RSD_TRY(st.sent(k, s));
+  }
   return RSD_OK;
 }
 
@@ -273,7 +455,7 @@ static int h2d_block(const double* h, int ldh, double* ddst, int ldd, int m, int
 // src(n x n, ld lds) -> dst(n x n, ld ldd).  Returns INFO >= 0 or an error.
 static int matrev_device(DenseWork& w, const double* src, int n, int lds, double* dst, int ldd, hipStream_t s) {
   const int np = round_up(std::max(n, 1), kTile);
-  DBuf A, Ai;
+  ArenaBuf A, Ai;
   RSD_TRY(A.alloc((size_t)np * np));
   RSD_TRY(Ai.alloc((size_t)np * np));
   RSD_TRY(dense_reserve(w, np, s));
@@ -403,14 +585,15 @@ static int per_grpery_impl(int n, const double* pos, const double* radii, rsd_la
   }
   const int n11 = 11 * n, n6 = 6 * n, n5 = 5 * n;
   hipStream_t s = nullptr;
-  DBuf dpos, drad, G, kw;
-  int* dov = nullptr;
+  ArenaBuf dpos, drad, G, kw;
+  ArenaBuf ov;
   RSD_TRY(dpos.alloc(3 * (size_t)n));
   RSD_TRY(drad.alloc(n));
   RSD_TRY(G.alloc((size_t)n11 * n11));
   const int side = 2 * lat->ni + 1;
   RSD_TRY(kw.alloc((size_t)side * side * side * rsdm::kKW));
-  RSD_HIP(hipMalloc(&dov, sizeof(int)));
+  RSD_TRY(ov.alloc(1));
+  int* dov = reinterpret_cast<int*>(ov.p);
   RSD_HIP(hipMemsetAsync(dov, 0, sizeof(int), s));
   RSD_HIP(hipMemcpyAsync(dpos.p, pos, 3 * (size_t)n * sizeof(double), hipMemcpyHostToDevice, s));
   RSD_HIP(hipMemcpyAsync(drad.p, radii, (size_t)n * sizeof(double), hipMemcpyHostToDevice, s));
@@ -426,7 +609,6 @@ static int per_grpery_impl(int n, const double* pos, const double* radii, rsd_la
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) rc = hip_fail(e, "per_grpery_inv_fri sync", __FILE__, __LINE__);
   }
-  (void)hipFree(dov);
   if (n_overlap) *n_overlap = nov;
   return rc;
 }
@@ -476,12 +658,13 @@ int rsd_grpery_inv_fri(int n, const double* pos, const double* radii, int correc
   if (n < 1 || !pos || !radii || !app || !apq || !aqq || !(mu_f > 0.0)) return RSD_ERR_ARG;
   const int n11 = 11 * n, n6 = 6 * n, n5 = 5 * n;
   hipStream_t s = nullptr;
-  DBuf dpos, drad, G;
-  int* dov = nullptr;
+  ArenaBuf dpos, drad, G;
+  ArenaBuf ov;
   RSD_TRY(dpos.alloc(3 * (size_t)n));
   RSD_TRY(drad.alloc(n));
   RSD_TRY(G.alloc((size_t)n11 * n11));
-  RSD_HIP(hipMalloc(&dov, sizeof(int)));
+  RSD_TRY(ov.alloc(1));
+  int* dov = reinterpret_cast<int*>(ov.p);
   RSD_HIP(hipMemsetAsync(dov, 0, sizeof(int), s));
   RSD_HIP(hipMemcpyAsync(dpos.p, pos, 3 * (size_t)n * sizeof(double), hipMemcpyHostToDevice, s));
   RSD_HIP(hipMemcpyAsync(drad.p, radii, (size_t)n * sizeof(double), hipMemcpyHostToDevice, s));
@@ -496,7 +679,6 @@ int rsd_grpery_inv_fri(int n, const double* pos, const double* radii, int correc
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) rc = hip_fail(e, "grpery_inv_fri sync", __FILE__, __LINE__);
   }
-  (void)hipFree(dov);
   if (n_overlap) *n_overlap = nov;
   return rc;
 }
@@ -505,7 +687,7 @@ int rsd_wall_grpery_inv_fri(int n, const double* pos, const double* radii, doubl
   if (n < 1 || !pos || !radii || !tpp || !(mu_f > 0.0)) return RSD_ERR_ARG;
   const int n3 = 3 * n;
   hipStream_t s = nullptr;
-  DBuf dpos, drad, T;
+  ArenaBuf dpos, drad, T;
   RSD_TRY(dpos.alloc(3 * (size_t)n));
   RSD_TRY(drad.alloc(n));
   RSD_TRY(T.alloc((size_t)n3 * n3));
@@ -524,14 +706,15 @@ int rsd_lubmxcalc(int n, int nb, int is_period, const double* pos, const double*
   RSD_TRY(device_tables(&tab));
   const int n6 = 6 * n, n5 = 5 * n;
   hipStream_t s = nullptr;
-  DBuf dpos, drad, dpp, dpq, dqq;
+  ArenaBuf dpos, drad, dpp, dpq, dqq;
   RSD_TRY(dpos.alloc(3 * (size_t)n));
   RSD_TRY(drad.alloc(n));
   RSD_TRY(dpp.alloc((size_t)n6 * n6));
   RSD_TRY(dpq.alloc((size_t)n6 * n5));
   RSD_TRY(dqq.alloc((size_t)n5 * n5));
-  int* dct = nullptr;
-  RSD_HIP(hipMalloc(&dct, sizeof(int)));
+  ArenaBuf ct;
+  RSD_TRY(ct.alloc(1));
+  int* dct = reinterpret_cast<int*>(ct.p);
   RSD_HIP(hipMemsetAsync(dct, 0, sizeof(int), s));
   RSD_HIP(hipMemcpyAsync(dpos.p, pos, 3 * (size_t)n * sizeof(double), hipMemcpyHostToDevice, s));
   RSD_HIP(hipMemcpyAsync(drad.p, radii, (size_t)n * sizeof(double), hipMemcpyHostToDevice, s));
@@ -562,7 +745,6 @@ int rsd_lubmxcalc(int n, int nb, int is_period, const double* pos, const double*
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) rc = hip_fail(e, "lubmxcalc sync", __FILE__, __LINE__);
   }
-  (void)hipFree(dct);
   if (n_contact) *n_contact = nc;
   return rc;
 }
@@ -575,7 +757,7 @@ static DenseWork& host_api_dense() {
 int rsd_matrev(int n, double* a) {
   if (n < 1 || !a) return RSD_ERR_ARG;
   hipStream_t s = nullptr;
-  DBuf A;
+  ArenaBuf A;
   RSD_TRY(A.alloc((size_t)n * n));
   RSD_TRY(h2d_block(a, n, A.p, n, n, n, s));
   int info = matrev_device(host_api_dense(), A.p, n, n, A.p, n, s);
@@ -590,7 +772,7 @@ int rsd_cholesky(int n, double* a) {
   const int np = round_up(n, kTile);
   hipStream_t s = nullptr;
   DenseWork& w = host_api_dense();
-  DBuf A;
+  ArenaBuf A;
   RSD_TRY(A.alloc((size_t)np * np));
   RSD_TRY(h2d_block(a, n, A.p, np, n, n, s));
   RSD_TRY(set_identity_padding(A.p, n, np, np, s));
@@ -616,7 +798,7 @@ int rsd_mob_to_resist_fts(int n, const double* app, const double* apq, const dou
   if (n < 1 || !app || !apq || !aqq || !rpp || !rpq || !rqq) return RSD_ERR_ARG;
   const int n11 = 11 * n, n6 = 6 * n, n5 = 5 * n;
   hipStream_t s = nullptr;
-  DBuf M;
+  ArenaBuf M;
   RSD_TRY(M.alloc((size_t)n11 * n11));
   // matrices.f90:400-403: [APP APQ; APQ^T AQQ]; only the upper triangle is read
   RSD_TRY(h2d_block(app, n6, M.p, n11, n6, n6, s));
@@ -636,7 +818,7 @@ static int arrangement_device(DenseWork& w, const double* dRPP, const double* dR
                               double* dMU, hipStream_t s) {
   const int n6 = 6 * n, n5 = 5 * n;
   const int n6p = round_up(n6, kTile), n5p = round_up(n5, kTile);
-  DBuf Pi, Qp, T, Mu;
+  ArenaBuf Pi, Qp, T, Mu;
   RSD_TRY(Pi.alloc((size_t)n6p * n6p));
   RSD_TRY(Qp.alloc((size_t)n6p * n5p));
   RSD_TRY(T.alloc((size_t)n6p * n5p));
@@ -682,7 +864,7 @@ int rsd_arrangement(int n, const double* rpp, const double* rpq, const double* r
   if (n < 1 || !rpp || !rpq || !rqq || !mu) return RSD_ERR_ARG;
   const int n6 = 6 * n, n5 = 5 * n;
   hipStream_t s = nullptr;
-  DBuf P, Q, R, M;
+  ArenaBuf P, Q, R, M;
   RSD_TRY(P.alloc((size_t)n6 * n6));
   RSD_TRY(Q.alloc((size_t)n6 * n5));
   RSD_TRY(R.alloc((size_t)n5 * n5));
@@ -707,16 +889,16 @@ extern "C" int rsd_stepper_nogmres(int n, const double* app, const double* apq, 
   const int n11 = 11 * n, n6 = 6 * n, n5 = 5 * n;
   hipStream_t s = nullptr;
   DenseWork& w = host_api_dense();
-  DBuf M, RPP, RPQ, RQQ, APPR, MU, vfe, vein, vc, vu, vs;
+  ArenaBuf M, RPP, RPQ, RQQ, APPR, vfe, vein, vc, vq, vu, vs;
   RSD_TRY(M.alloc((size_t)n11 * n11));
   RSD_TRY(RPP.alloc((size_t)n6 * n6));
   RSD_TRY(RPQ.alloc((size_t)n6 * n5));
   RSD_TRY(RQQ.alloc((size_t)n5 * n5));
   RSD_TRY(APPR.alloc((size_t)n6 * n6));
-  RSD_TRY(MU.alloc((size_t)n5 * n5));
   RSD_TRY(vfe.alloc(n6));
   RSD_TRY(vein.alloc(n5));
   RSD_TRY(vc.alloc(n6));
+  RSD_TRY(vq.alloc(n6));
   RSD_TRY(vu.alloc(n6));
   RSD_TRY(vs.alloc(n5));
   // MobToResist_FTS (matrices.f90:393-416)
@@ -729,7 +911,7 @@ extern "C" int rsd_stepper_nogmres(int n, const double* app, const double* apq, 
   RSD_TRY(copy_block(M.p, n11, RPP.p, n6, n6, n6, s));
   RSD_TRY(copy_block(M.p + (size_t)n6 * n11, n11, RPQ.p, n6, n6, n5, s));
   RSD_TRY(copy_block(M.p + n6 + (size_t)n6 * n11, n11, RQQ.p, n5, n5, n5, s));
-  DBuf L;
+  ArenaBuf L;
   RSD_TRY(L.alloc((size_t)n6 * n6));
   RSD_TRY(h2d_block(rfu, n6, L.p, n6, n6, n6, s));
   RSD_TRY(matrix_axpy(1.0, L.p, n6, RPP.p, n6, n6, n6, s));
@@ -737,23 +919,24 @@ extern "C" int rsd_stepper_nogmres(int n, const double* app, const double* apq, 
   RSD_TRY(matrix_axpy(1.0, L.p, n6, RPQ.p, n6, n6, n5, s));
   RSD_TRY(h2d_block(rse, n5, L.p, n5, n5, n5, s));
   RSD_TRY(matrix_axpy(1.0, L.p, n5, RQQ.p, n5, n5, n5, s));
-  // U_par = inv(RPP) (Fe + RPQ EIN)   (stepper.f90:387-395)
+  // U_par = inv(RPP) (Fe + RPQ EIN)   (stepper.f90:387-395) and
+  // SijN_hyd = mu EIN, mu = RPQ^T inv(RPP) RPQ - RQQ   (stepper.f90:401-403),
+  // mu only in its product with EIN
   int info2 = matrev_device(w, RPP.p, n6, n6, APPR.p, n6, s);
   if (info2 < 0) return info2;
-  RSD_HIP(hipMemcpyAsync(vfe.p, fe, n6 * sizeof(double), hipMemcpyHostToDevice, s));
-  RSD_HIP(hipMemcpyAsync(vein.p, ein, n5 * sizeof(double), hipMemcpyHostToDevice, s));
-  RSD_HIP(hipMemcpyAsync(vc.p, vfe.p, n6 * sizeof(double), hipMemcpyDeviceToDevice, s));
-  RSD_TRY(gemv(w, RPQ.p, n6, n6, n5, false, 1.0, vein.p, 1.0, vc.p, s));
+  RSD_TRY(h2d_block(fe, n6, vfe.p, n6, n6, 1, s));
+  RSD_TRY(h2d_block(ein, n5, vein.p, n5, n5, 1, s));
+  RSD_TRY(gemv(w, RPQ.p, n6, n6, n5, false, 1.0, vein.p, 0.0, vq.p, s));
+  RSD_TRY(vector_sum(vfe.p, vq.p, vc.p, n6, s));
   RSD_TRY(gemv(w, APPR.p, n6, n6, n6, false, 1.0, vc.p, 0.0, vu.p, s));
-  // SijN_hyd = mu EIN, mu = RPQ^T inv(RPP) RPQ - RQQ   (stepper.f90:401-403)
-  int info3 = arrangement_device(w, RPP.p, RPQ.p, RQQ.p, n, MU.p, s);
-  if (info3 < 0) return info3;
-  RSD_TRY(gemv(w, MU.p, n5, n5, n5, false, 1.0, vein.p, 0.0, vs.p, s));
-  RSD_HIP(hipMemcpyAsync(u_par, vu.p, n6 * sizeof(double), hipMemcpyDeviceToHost, s));
-  RSD_HIP(hipMemcpyAsync(sijn_hyd, vs.p, n5 * sizeof(double), hipMemcpyDeviceToHost, s));
+  RSD_TRY(gemv(w, APPR.p, n6, n6, n6, false, 1.0, vq.p, 0.0, vc.p, s));
+  RSD_TRY(gemv(w, RPQ.p, n6, n6, n5, true, 1.0, vc.p, 0.0, vs.p, s));
+  RSD_TRY(gemv(w, RQQ.p, n5, n5, n5, false, -1.0, vein.p, 1.0, vs.p, s));
+  RSD_TRY(d2h_block(vu.p, n6, u_par, n6, n6, 1, s));
+  RSD_TRY(d2h_block(vs.p, n5, sijn_hyd, n5, n5, 1, s));
   if (rpp) RSD_TRY(d2h_block(RPP.p, n6, rpp, n6, n6, n6, s));
   RSD_HIP(hipStreamSynchronize(s));
-  return info ? info : (info2 ? info2 : info3);
+  return info ? info : info2;
 }
 
 // ===================================================== device-resident step

@@ -860,7 +860,7 @@ __device__ __forceinline__ void diag_factor64(double (&a)[16], DiagSmem& sm, int
 
 // the inverse (column-major, zero upper blocks; written through) and the INFO word
 __device__ __forceinline__ void diag_store_inverse(const DiagSmem& sm, double* __restrict__ dinv, int* __restrict__ info) {
-  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63;
+  const int tid = opaque_tid(), w = tid >> 6, l = tid & 63;
 #pragma unroll
   for (int q = 0; q < 16; ++q) {
     const int c = 16 * w + q;
@@ -871,7 +871,7 @@ __device__ __forceinline__ void diag_store_inverse(const DiagSmem& sm, double* _
 
 // the factor into the matrix at (k0, k0)
 __device__ __forceinline__ void diag_store_factor(const DiagSmem& sm, double* __restrict__ A, int ld, int k0) {
-  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63;
+  const int tid = opaque_tid(), w = tid >> 6, l = tid & 63;
 #pragma unroll
   for (int q = 0; q < 16; ++q) {
     const int c = 16 * w + q;
@@ -978,6 +978,7 @@ struct DagArgs {
   int* sync;     // [0] ticket, [1] error word, [2, 2+nt*nt) tile flags, then 2 nt partial
                  // flags, then (with X) ns*ns flags of X's tiles
   int gen;
+  int nfac;      // the factorization's tickets after the walker's
   int* info;
   int* rec;      // the first timed-out wait: [1, ticket, flag index, flag value]
   // optional: X = inv(L_S) of the trailing block L_S (tiles s0..nt-1, ns = nt - s0
@@ -1250,6 +1251,341 @@ __device__ __forceinline__ void pair_accumulate(v4d (&acc)[2][2], const Terms& T
   __syncthreads();  // the staging buffers are free again
 }
 
+// ------------------------------------------------ macro tasks (large matrices)
+// A macro task is two block rows by two block columns of the factor, a 128x128
+// tile, accumulated as one: each wave keeps a 64x64 tile of it.  A 64-deep term
+// of four tiles then moves 128 KB into LDS where four single tiles move 256 KB,
+// and past N ~ 700 those reads (L2 misses, 5.2 TB/s) are what bounds the
+// single-tile tasks.  A term is two 32-column halves through two LDS buffers;
+// an 8-step half keeps the matrix cores busy for 8192 cycles, its one barrier
+// is before its last step, and each step's operands are read during the step
+// before it.  Both factorisations of a step: N = 4096 815 -> 617 ms (57 TF/s),
+// N = 2048 99 -> 83 ms.
+struct MacroOps {
+  double a[4], b[4];
+};
+// a lane's operands of step 0 in a buffer (T1's 128 rows x 32 columns, then T2's, laid out as stage_macro does)
+struct MacroAt {
+  int a[4], b[4];
+};
+__device__ __forceinline__ MacroAt macro_at() {
+  const int tid = opaque_tid(), lane = tid & 63, wave = tid >> 6;
+  const int m = lane & 15, kq = lane >> 4, swap = (kq & 1) << 4;
+  MacroAt at;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    at.a[q] = kq * 128 + ((64 * (wave & 1) + 16 * q + m) ^ swap);
+    at.b[q] = 4096 + kq * 128 + ((64 * (wave >> 1) + 16 * q + m) ^ swap);
+  }
+  return at;
+}
+// a quarter of the reads, and of a step's products (its 16 MFMAs by rows)
+__device__ __forceinline__ void macro_read(MacroOps& o, const MacroAt& at, int u, int q, const double* buf) {
+  const double* b = buf + 512 * u;
+  o.a[q] = b[at.a[q]];
+  o.b[q] = b[at.b[q]];
+}
+__device__ __forceinline__ void macro_mfma(v4d (&nacc)[4][4], const MacroOps& o, int bm) {
+#pragma unroll
+  for (int bn = 0; bn < 4; ++bn)
+    nacc[bm][bn] = __builtin_amdgcn_mfma_f64_16x16x4f64(o.a[bm], o.b[bn], nacc[bm][bn], 0, 0, 0);
+}
+// this wave's q-th (of 8) direct load of a 128x32 chunk: column 8 wave + q, its
+// 16-row blocks swapped in pairs on odd columns (as staged())
+__device__ __forceinline__ void macro_load(const double* p, int ld, int lane, int q, double* dst) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = 8 * wave + q;
+  const unsigned at = 2 * (lane ^ ((q & 1) << 3));
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(p + (size_t)c * ld + at),
+                                   (__attribute__((address_space(3))) void*)(dst + c * 128), 16, 0, kCpolSc1);
+}
+// steps 0..6 of the half at rd (its step 0 in P; step 7 is left in Q), with the
+// loads of the next half into wr (ST): two reads and, in the first four steps,
+// one load between every four MFMAs.  (All 16 loads in front of the half's
+// products, the matrix cores idle until they are issued: N = 4096's step took
+// 993 ms so, 934 with eight in each of two steps, 924 with four in each of four.)
+template <bool ST>
+__device__ __forceinline__ void macro_half(v4d (&nacc)[4][4], MacroOps& P, MacroOps& Q, const MacroAt& at,
+                                           const double* __restrict__ rd, const double* __restrict__ t1,
+                                           const double* __restrict__ t2, int ld, double* __restrict__ wr) {
+  const int lane = ST ? opaque_tid() & 63 : 0;
+#pragma unroll
+  for (int u = 0; u < 7; ++u)
+#pragma unroll
+    for (int bm = 0; bm < 4; ++bm) {
+      macro_read(u & 1 ? P : Q, at, u + 1, bm, rd);
+      if (ST && u < 4) macro_load(bm & 1 ? t2 : t1, ld, lane, 2 * u + (bm >> 1), bm & 1 ? wr + 4096 : wr);
+      macro_mfma(nacc, u & 1 ? Q : P, bm);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// nacc += sum_{k < kend} T1_k T2_k^T, T1_k the 128 rows at p1 + 64 k ld (block
+// rows i0, i0 + 1 of the factor), T2_k those at p2 (block rows j0, j0 + 1); each
+// term once its four tiles are published
+__device__ __forceinline__ void macro_accumulate(v4d (&nacc)[4][4], int kend, const double* p1, const double* p2, int ld,
+                                                 int nt, int i0, int j0, const int* flags, int gen, int* err,
+                                                 double* smem, int* rec, int who) {
+  if (kend <= 0) return;
+  const int lane = opaque_tid() & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int* kready_x = reinterpret_cast<int*>(smem + kDagSmemDoubles) + 1;
+  int kready = 0;
+  auto load = [&](int f) { return __hip_atomic_load(&flags[f], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+  auto first_not = [&](int k, bool ok) {
+    const unsigned long long no = ~__ballot(ok);
+    return k + (no ? __builtin_ctzll(no) : 64);
+  };
+  auto ready = [&](int k) {
+    if (wave == 0) {
+      bool ok = false;
+      if (k + lane < kend) {
+        const int c = nt * (k + lane);
+        const int v1 = load(i0 + c), v2 = load(i0 + 1 + c), v3 = load(j0 + c), v4 = load(j0 + 1 + c);
+        ok = v1 == gen && v2 == gen && v3 == gen && v4 == gen;
+      }
+      int kk = first_not(k, ok);
+      if (kk == k) {
+        if (lane == 0) {
+          const int c = nt * k;
+          for (int f : {i0 + c, i0 + 1 + c, j0 + c, j0 + 1 + c}) wait_flag(&flags[f], gen, err, rec, who, f);
+        }
+        kk = k + 1;
+      }
+      if (lane == 0) kready_x[2] = kk;
+    }
+    __syncthreads();
+    kready = __builtin_amdgcn_readfirstlane(kready_x[2]);
+    wt_seen();
+  };
+  auto buffer = [&](int h) { return smem + (h & 1) * 8192; };
+  const MacroAt at = macro_at();
+  MacroOps P, Q;
+  int issued;  // halves before it are staged or on their way
+  auto restart = [&](int h) {
+    ready(h >> 1);
+    const size_t col = (size_t)(32 * h) * ld;
+    const int ln = opaque_tid() & 63;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      macro_load(p1 + col, ld, ln, q, buffer(h));
+      macro_load(p2 + col, ld, ln, q, buffer(h) + 4096);
+    }
+    issued = h + 1;
+    __builtin_amdgcn_s_waitcnt(kWaitVm0);
+    gemm_barrier();
+#pragma unroll
+    for (int q = 0; q < 4; ++q) macro_read(P, at, 0, q, buffer(h));
+  };
+  auto last_step = [&] {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) macro_mfma(nacc, Q, q);
+  };
+  restart(0);
+  const int halves = 2 * kend;
+  for (int h = 0; h < halves; ++h) {
+    const bool scan = kready < kend && kready <= (h >> 1) + 2;
+    int v1 = gen, v2 = gen, v3 = gen, v4 = gen;
+    if (scan) {
+      const int c = nt * min(kready + lane, kend - 1);
+      v1 = load(i0 + c);
+      v2 = load(i0 + 1 + c);
+      v3 = load(j0 + c);
+      v4 = load(j0 + 1 + c);
+    }
+    if (issued == h + 1 && h + 1 < halves && (h + 1) >> 1 < kready) {
+      const size_t col = (size_t)(32 * (h + 1)) * ld;
+      macro_half<true>(nacc, P, Q, at, buffer(h), p1 + col, p2 + col, ld, buffer(h + 1));
+      issued = h + 2;
+    } else {
+      macro_half<false>(nacc, P, Q, at, buffer(h), nullptr, nullptr, 0, buffer(h + 1));
+    }
+    if (h + 1 == halves) {
+      last_step();
+      break;
+    }
+    __builtin_amdgcn_s_waitcnt(kWaitVm0);  // this wave's share of half h+1 has landed
+    if (scan) {
+      asm volatile("" : "+v"(v1), "+v"(v2), "+v"(v3), "+v"(v4));  // (compared here, not where they were loaded)
+      const int kk = first_not(kready, kready + lane < kend && v1 == gen && v2 == gen && v3 == gen && v4 == gen);
+      if (threadIdx.x == 0) kready_x[h & 1] = kk;
+    }
+    gemm_barrier();
+    if (scan) {
+      kready = __builtin_amdgcn_readfirstlane(kready_x[h & 1]);
+      wt_seen();
+    }
+    if (issued <= h + 1) {
+      last_step();
+      restart(h + 1);
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        macro_read(P, at, 0, q, buffer(h + 1));
+        macro_mfma(nacc, Q, q);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  }
+  __syncthreads();  // the staging buffers are free again
+}
+
+// LDS of a macro task's end: a 128x64 block by columns (Cs[kk][m], m < 128),
+// then a staged 64x64 tile.  A wave owns rows 32 wave..32 wave + 31 of the block.
+constexpr int kMacroLd = 130;
+static_assert(64 * kMacroLd + 4096 <= kDagSmemDoubles, "a macro task's end fits the shared buffer");
+// acc += C T^T for this wave's 32 rows of the block in Cs and the staged tile T
+__device__ __forceinline__ void macro_rows_product(v4d (&acc)[2][4], const double* Cs, const double* T) {
+  const int tid = opaque_tid(), lane = tid & 63, wave = tid >> 6, m = lane & 15;
+#pragma unroll
+  for (int st = 0; st < 16; ++st) {
+    const int kr = 4 * st + (lane >> 4);
+    const double a0 = Cs[kr * kMacroLd + 32 * wave + m], a1 = Cs[kr * kMacroLd + 32 * wave + 16 + m];
+#pragma unroll
+    for (int bn = 0; bn < 4; ++bn) {
+      const double b = T[staged(16 * bn + m, kr)];
+      acc[0][bn] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b, acc[0][bn], 0, 0, 0);
+      acc[1][bn] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b, acc[1][bn], 0, 0, 0);
+    }
+  }
+}
+// this wave's rows of the block, accumulator layout <-> Cs; sign: of what is written
+__device__ __forceinline__ void macro_rows_put(const v4d (&x)[2][4], double* Cs, double sign) {
+  const int tid = opaque_tid(), lane = tid & 63, wave = tid >> 6;
+#pragma unroll
+  for (int bm = 0; bm < 2; ++bm)
+#pragma unroll
+    for (int bn = 0; bn < 4; ++bn)
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+        Cs[(16 * bn + (lane & 15)) * kMacroLd + 32 * wave + 16 * bm + (lane >> 4) + 4 * v] = sign * x[bm][bn][v];
+  wave_lds_order();
+}
+// this wave's rows of the block in Cs out to dst (written through), 256-byte column pieces
+__device__ __forceinline__ void macro_rows_store(const double* Cs, double* dst, size_t ld) {
+  const int tid = opaque_tid(), lane = tid & 63, wave = tid >> 6;
+#pragma unroll
+  for (int it = 0; it < 16; ++it) {
+    const int c = 4 * it + (lane >> 4), r = 32 * wave + 2 * (lane & 15);
+    const double2 x = *reinterpret_cast<const double2*>(&Cs[c * kMacroLd + r]);
+    wt_store(dst + (size_t)r + (size_t)c * ld, x.x);
+    wt_store(dst + (size_t)r + 1 + (size_t)c * ld, x.y);
+  }
+}
+
+// The macro task (I, J): block rows 2I, 2I + 1 of block columns 2J, 2J + 1
+__device__ __forceinline__ void macro_task(const DagArgs& g, int I, int J, int t, double* __restrict__ smem) {
+  const int tid = opaque_tid(), lane = tid & 63, wave = tid >> 6, nt = g.nt, ld = g.ld;
+  const int i0 = 2 * I, j0 = 2 * J;
+  int* err = g.sync + 1;
+  int* flags = g.sync + 2;
+  double* tile = g.A + 64 * i0 + (size_t)(64 * j0) * ld;
+  double* Cs = smem;
+  double* Dj = smem + 64 * kMacroLd;
+  v4d d1[2][4];  // this wave's rows of the second block column, negated
+  {
+    const int wm = 64 * (wave & 1), wn = 64 * (wave >> 1);
+    v4d acc[4][4];  // negated: the terms add to it
+#pragma unroll
+    for (int bm = 0; bm < 4; ++bm)
+#pragma unroll
+      for (int bn = 0; bn < 4; ++bn)
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+          acc[bm][bn][v] = -tile[(size_t)(wm + 16 * bm + (lane >> 4) + 4 * v) +
+                                 (size_t)(wn + 16 * bn + (lane & 15)) * ld];
+    macro_accumulate(acc, j0, g.A + 64 * i0, g.A + 64 * j0, ld, nt, i0, j0, flags, g.gen, err, smem, g.rec, t);
+    // the two block columns through Cs, from a 64x64 tile a wave to 32 rows a wave
+    auto put = [&](double sign) {
+#pragma unroll
+      for (int bm = 0; bm < 4; ++bm)
+#pragma unroll
+        for (int bn = 0; bn < 4; ++bn)
+#pragma unroll
+          for (int v = 0; v < 4; ++v)
+            Cs[(16 * bn + (lane & 15)) * kMacroLd + wm + 16 * bm + (lane >> 4) + 4 * v] = sign * acc[bm][bn][v];
+    };
+    if (wave >> 1) put(1.0);
+    __syncthreads();
+#pragma unroll
+    for (int bm = 0; bm < 2; ++bm)
+#pragma unroll
+      for (int bn = 0; bn < 4; ++bn)
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+          d1[bm][bn][v] = Cs[(16 * bn + (lane & 15)) * kMacroLd + 32 * wave + 16 * bm + (lane >> 4) + 4 * v];
+    __syncthreads();
+    if (!(wave >> 1)) put(-1.0);
+  }
+  // a published tile into Dj, once its flag is up (and every wave is past its
+  // use of Dj and, the first time, has written Cs)
+  auto fetch = [&](int f, const double* src, int sld) {
+    if (tid == 0) wait_flag(&flags[f], g.gen, err, g.rec, t, f);
+    __syncthreads();
+    wt_seen();
+    stage_tile(src, sld, Dj);
+    __builtin_amdgcn_s_waitcnt(kWaitVm0);
+    __syncthreads();
+  };
+  auto publish = [&](int j) {
+    wt_stores_done();
+    __syncthreads();
+    if (tid == 0) {
+      wt_publish(&flags[i0 + nt * j], g.gen);
+      wt_publish(&flags[i0 + 1 + nt * j], g.gen);
+    }
+  };
+  v4d out[2][4];
+  auto clear = [&] {
+#pragma unroll
+    for (int bm = 0; bm < 2; ++bm)
+#pragma unroll
+      for (int bn = 0; bn < 4; ++bn) out[bm][bn] = (v4d){0.0, 0.0, 0.0, 0.0};
+  };
+  // L of the first block column
+  fetch(j0 + nt * j0, g.dinv + (size_t)j0 * 4096, 64);
+  clear();
+  macro_rows_product(out, Cs, Dj);
+  wave_lds_order();
+  macro_rows_put(out, Cs, 1.0);
+  macro_rows_store(Cs, tile, ld);
+  publish(j0);
+  // its term of the second, and L of that
+  fetch(j0 + 1 + nt * j0, g.A + 64 * (j0 + 1) + (size_t)(64 * j0) * ld, ld);
+  macro_rows_product(d1, Cs, Dj);
+  wave_lds_order();
+  macro_rows_put(d1, Cs, -1.0);
+  fetch(j0 + 1 + nt * (j0 + 1), g.dinv + (size_t)(j0 + 1) * 4096, 64);
+  clear();
+  macro_rows_product(out, Cs, Dj);
+  wave_lds_order();
+  macro_rows_put(out, Cs, 1.0);
+  macro_rows_store(Cs, tile + (size_t)64 * ld, ld);
+  publish(j0 + 1);
+}
+
+// Ticket order with macro tasks, per pair J of block columns: the early tiles
+// of columns 2J + kAhead and 2J + 1 + kAhead; tile (2J+3, 2J) alone; the macro
+// tasks (I, J), I >= J + 2; and, when nt is odd, the last block row's two tiles.
+struct MacroCounts {
+  int e0, e1, single, macros, last;
+};
+__host__ __device__ inline int dag_early(int nt, int c) { return c < nt ? (kEarly < nt - c ? kEarly : nt - c) : 0; }
+__host__ __device__ inline MacroCounts macro_counts(int nt, int J) {
+  const int m = nt / 2 - (J + 2);
+  return {dag_early(nt, 2 * J + kAhead), dag_early(nt, 2 * J + 1 + kAhead), 2 * J + 3 < nt ? 1 : 0, m > 0 ? m : 0,
+          (nt & 1) && nt - 1 >= 2 * J + 4 ? 2 : 0};
+}
+// the factorization's tickets after the walker's
+static int dag_tickets(int nt, bool macro) {
+  if (!macro) return nt * (nt + 1) / 2;
+  int n = 0;
+  for (int c = 0; c < kAhead; ++c) n += dag_early(nt, c);
+  for (int J = 0; J < (nt + 1) / 2; ++J) {
+    const MacroCounts k = macro_counts(nt, J);
+    n += k.e0 + k.e1 + k.single + k.macros + k.last;
+  }
+  return n;
+}
+
 // out = acc Dinv^T, Dinv a column-major 64x64 tile in global memory
 __device__ __forceinline__ void tile_trsm(const v4d (&acc)[2][2], const double* __restrict__ Dg, double* smem,
                                           v4d (&out)[2][2]) {
@@ -1390,9 +1726,8 @@ __device__ __forceinline__ void walker_lt_product(v4d (&Lt)[2][2], const double 
   }
 }
 
-// One task of the dataflow Cholesky: ticket 0 the walker, the others a tile
-// (see above).  Returns when the task is done.
-__device__ __forceinline__ void dag_task(const DagArgs& g, int t, double* __restrict__ smem) {
+// The walker (ticket 0; see above)
+__device__ __forceinline__ void dag_walker(const DagArgs& g, double* __restrict__ smem) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
   const int nt = g.nt, ld = g.ld;
@@ -1402,91 +1737,101 @@ __device__ __forceinline__ void dag_task(const DagArgs& g, int t, double* __rest
   int* pflags = g.sync + 2 + nt * nt;
   int* rec = g.rec;  // the first timed-out wait
   v4d acc[2][2];
-
-  if (t == 0) {  // the walker
-    // acc: partial sum of the current diagonal tile, already including the
-    // last update (the previous column's L_{j,j-1} L_{j,j-1}^T)
-    DiagSmem& sm = *reinterpret_cast<DiagSmem*>(smem);
-    if (tid == 0) wait_flag(&pflags[0], g.gen, err, rec, 0, nt * nt);
+  // acc: partial sum of the current diagonal tile, already including the
+  // last update (the previous column's L_{j,j-1} L_{j,j-1}^T)
+  DiagSmem& sm = *reinterpret_cast<DiagSmem*>(smem);
+  if (tid == 0) wait_flag(&pflags[0], g.gen, err, rec, 0, nt * nt);
+  __syncthreads();
+  wt_seen();
+  tile_load<true>(acc, g.part, 64);
+  for (int j = 0; j < nt; ++j) {
+#pragma unroll
+    for (int bm = 0; bm < 2; ++bm)
+#pragma unroll
+      for (int bn = 0; bn < 2; ++bn)
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+          sm.Ls[wm + 16 * bm + (lane >> 4) + 4 * v][wn + 16 * bn + (lane & 15)] = acc[bm][bn][v];
     __syncthreads();
-    wt_seen();
-    tile_load<true>(acc, g.part, 64);
-    for (int j = 0; j < nt; ++j) {
+    double a[16];
 #pragma unroll
-      for (int bm = 0; bm < 2; ++bm)
-#pragma unroll
-        for (int bn = 0; bn < 2; ++bn)
-#pragma unroll
-          for (int v = 0; v < 4; ++v)
-            sm.Ls[wm + 16 * bm + (lane >> 4) + 4 * v][wn + 16 * bn + (lane & 15)] = acc[bm][bn][v];
-      __syncthreads();
-      double a[16];
-#pragma unroll
-      for (int q = 0; q < 16; ++q) a[q] = sm.Ls[lane][16 * wave + q];
-      __syncthreads();
-      // column j+1's partial tiles, (j+1,j) into sa0/sa1 (the A operands of
-      // L_{j+1,j}'s product) and (j+1,j+1) into acc: each wave issues its
-      // share of the loads at the first point where both are published (the
-      // column's start, or a point of slack in the factorization), so that
-      // they land during it; a wave that has not issued them by the end of
-      // the factorization waits for the tiles there.  The loads go to
-      // registers: loads into LDS would hold up every barrier until they land.
-      double sa0[16], sa1[16];
-      const double* sub_src = g.part + (size_t)(2 * j + 1) * 4096;
-      const double* acc_src = g.part + (size_t)(2 * (j + 1)) * 4096;
-      bool issued = j + 1 >= nt;
-      auto issue = [&](bool wait) {
-        if (issued) return;
-        if (wait) {
-          if (lane == 0) {
-            wait_flag(&pflags[2 * j + 1], g.gen, err, rec, 0, nt * nt + 2 * j + 1);
-            wait_flag(&pflags[2 * (j + 1)], g.gen, err, rec, 0, nt * nt + 2 * (j + 1));
-          }
-        } else {
-          const int ready =
-              __hip_atomic_load(&pflags[2 * j + 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == g.gen &&
-              __hip_atomic_load(&pflags[2 * (j + 1)], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == g.gen;
-          if (!__builtin_amdgcn_readfirstlane(ready)) return;
+    for (int q = 0; q < 16; ++q) a[q] = sm.Ls[lane][16 * wave + q];
+    __syncthreads();
+    // column j+1's partial tiles, (j+1,j) into sa0/sa1 (the A operands of
+    // L_{j+1,j}'s product) and (j+1,j+1) into acc: each wave issues its
+    // share of the loads at the first point where both are published (the
+    // column's start, or a point of slack in the factorization), so that
+    // they land during it; a wave that has not issued them by the end of
+    // the factorization waits for the tiles there.  The loads go to
+    // registers: loads into LDS would hold up every barrier until they land.
+    double sa0[16], sa1[16];
+    const double* sub_src = g.part + (size_t)(2 * j + 1) * 4096;
+    const double* acc_src = g.part + (size_t)(2 * (j + 1)) * 4096;
+    bool issued = j + 1 >= nt;
+    auto issue = [&](bool wait) {
+      if (issued) return;
+      if (wait) {
+        if (lane == 0) {
+          wait_flag(&pflags[2 * j + 1], g.gen, err, rec, 0, nt * nt + 2 * j + 1);
+          wait_flag(&pflags[2 * (j + 1)], g.gen, err, rec, 0, nt * nt + 2 * (j + 1));
         }
-        wt_seen();
-        tile_load_a(sa0, sa1, sub_src);
-        tile_load<true>(acc, acc_src, 64);
-        issued = true;
-      };
-      issue(false);
-      // the previous column's L_{j,j-1}: published by the last wave, which
-      // waits for the first panel's pivots anyway (its stores are behind the
-      // barriers above)
-      if (j > 0 && tid == 192) wt_publish(&flags[j + nt * (j - 1)], g.gen);
-      diag_factor64(a, sm, 64 * j, [&](int) { issue(false); });
-      diag_store_inverse(sm, g.dinv + (size_t)j * 4096, g.info);
-      wt_stores_done();
-      __syncthreads();
-      if (tid == 0) wt_publish(&flags[j + nt * j], g.gen);
-      diag_store_factor(sm, A, ld, 64 * j);  // read by nobody in this launch
-      if (j + 1 == nt) break;
-      issue(true);
-      __builtin_amdgcn_s_waitcnt(kWaitVm0);
-      __syncthreads();
-      // L_{j+1,j} = P_{j+1,j} X^T with X = inv(L_jj) still in sm.Xs (lower
-      // blocks).  X^T is block upper triangular, so output column block c
-      // takes only the k-steps of blocks 0..c; waves 0,1 form column blocks
-      // 0 and 3, waves 2,3 blocks 1 and 2: 40 MFMAs each instead of 64
-      v4d Lt[2][2];
-      if (wave >> 1)
-        walker_lt_product<1, 2>(Lt, sa0, sa1, sm, lane);
-      else
-        walker_lt_product<0, 3>(Lt, sa0, sa1, sm, lane);
-      __syncthreads();
-      // L_{j+1,j} out (written through), and the last update of the next
-      // diagonal tile, the stores' completion waited for at the end
-      const int cb0 = (wave >> 1) ? 1 : 0, cb1 = (wave >> 1) ? 2 : 3;
-      tile_store_syrk(acc, Lt, cb0, cb1, A + 64 * (j + 1) + (size_t)(64 * j) * ld, ld, smem);
-      // L_{j+1,j} is published at the start of the next column by a wave
-      // that is idle there
-    }
-    return;
+      } else {
+        const int ready =
+            __hip_atomic_load(&pflags[2 * j + 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == g.gen &&
+            __hip_atomic_load(&pflags[2 * (j + 1)], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == g.gen;
+        if (!__builtin_amdgcn_readfirstlane(ready)) return;
+      }
+      wt_seen();
+      tile_load_a(sa0, sa1, sub_src);
+      tile_load<true>(acc, acc_src, 64);
+      issued = true;
+    };
+    issue(false);
+    // the previous column's L_{j,j-1}: published by the last wave, which
+    // waits for the first panel's pivots anyway (its stores are behind the
+    // barriers above)
+    if (j > 0 && tid == 192) wt_publish(&flags[j + nt * (j - 1)], g.gen);
+    diag_factor64(a, sm, 64 * j, [&](int) { issue(false); });
+    diag_store_inverse(sm, g.dinv + (size_t)j * 4096, g.info);
+    wt_stores_done();
+    __syncthreads();
+    if (tid == 0) wt_publish(&flags[j + nt * j], g.gen);
+    diag_store_factor(sm, A, ld, 64 * j);  // read by nobody in this launch
+    if (j + 1 == nt) break;
+    issue(true);
+    __builtin_amdgcn_s_waitcnt(kWaitVm0);
+    __syncthreads();
+    // L_{j+1,j} = P_{j+1,j} X^T with X = inv(L_jj) still in sm.Xs (lower
+    // blocks).  X^T is block upper triangular, so output column block c
+    // takes only the k-steps of blocks 0..c; waves 0,1 form column blocks
+    // 0 and 3, waves 2,3 blocks 1 and 2: 40 MFMAs each instead of 64
+    v4d Lt[2][2];
+    if (wave >> 1)
+      walker_lt_product<1, 2>(Lt, sa0, sa1, sm, lane);
+    else
+      walker_lt_product<0, 3>(Lt, sa0, sa1, sm, lane);
+    __syncthreads();
+    // L_{j+1,j} out (written through), and the last update of the next
+    // diagonal tile, the stores' completion waited for at the end
+    const int cb0 = (wave >> 1) ? 1 : 0, cb1 = (wave >> 1) ? 2 : 3;
+    tile_store_syrk(acc, Lt, cb0, cb1, A + 64 * (j + 1) + (size_t)(64 * j) * ld, ld, smem);
+    // L_{j+1,j} is published at the start of the next column by a wave
+    // that is idle there
   }
+}
+
+// One tile task of the dataflow Cholesky, t >= 1 (see above).  Returns when the
+// task is done.
+template <bool MACRO>
+__device__ __forceinline__ void dag_task(const DagArgs& g, int t, double* __restrict__ smem) {
+  const int tid = threadIdx.x;
+  const int nt = g.nt, ld = g.ld;
+  double* __restrict__ A = g.A;
+  int* err = g.sync + 1;
+  int* flags = g.sync + 2;
+  int* pflags = g.sync + 2 + nt * nt;
+  int* rec = g.rec;  // the first timed-out wait
+  v4d acc[2][2];
 
   // A tile task: the tile (i,j) of the factor, or (past the factorization's
   // tickets) the tile (xi,xj) of X = inv(L_S), I = s0 + xi (see potrf_lower_x)
@@ -1494,11 +1839,11 @@ __device__ __forceinline__ void dag_task(const DagArgs& g, int t, double* __rest
   const int s0 = g.s0, ns = nt - s0;
   double* X = g.X;
   const int ldx = g.ldx;
-  const bool is_x = t > nt * (nt + 1) / 2;
+  const bool is_x = t > g.nfac;
   int i, j;  // the tile; of X: (xi, xj)
   Terms T;
   if (is_x) {
-    const int r = t - nt * (nt + 1) / 2 - 1;
+    const int r = t - g.nfac - 1;
     double* xdT = g.part + (size_t)2 * nt * 4096;   // X_jj^T = Dinv^T of the diagonal blocks
     if (r < ns) {
       // diagonal block j: X_jj = Dinv_J into X (read by the LL^T product after
@@ -1534,18 +1879,45 @@ __device__ __forceinline__ void dag_task(const DagArgs& g, int t, double* __rest
     T = Terms{j, i, xdT + (size_t)j * 4096, X + 64 * j, A + 64 * I + (size_t)(64 * s0) * ld,
               64, ldx, ld, xf + ns * j, 1, I + nt * s0, nt};
   } else {
-    auto esize = [nt](int c) { return c < nt ? min(kEarly, nt - c) : 0; };  // early tiles of column c
     int r = t - 1, c0 = 0;
     for (; c0 < kAhead && c0 < nt; ++c0) {
-      if (r < esize(c0)) break;
-      r -= esize(c0);
+      if (r < dag_early(nt, c0)) break;
+      r -= dag_early(nt, c0);
     }
     if (c0 < kAhead && c0 < nt) {
       j = c0;
       i = c0 + r;
+    } else if (MACRO) {
+      i = j = 0;
+      for (int J = 0;; ++J) {
+        const MacroCounts k = macro_counts(nt, J);
+        if (r < k.e0 + k.e1) {
+          j = 2 * J + kAhead + (r < k.e0 ? 0 : 1);
+          i = j + (r < k.e0 ? r : r - k.e0);
+          break;
+        }
+        r -= k.e0 + k.e1;
+        if (r < k.single) {
+          j = 2 * J;
+          i = j + 3;
+          break;
+        }
+        r -= k.single;
+        if (r < k.macros) {
+          macro_task(g, J + 2 + r, J, t, smem);
+          return;
+        }
+        r -= k.macros;
+        if (r < k.last) {
+          j = 2 * J + r;
+          i = nt - 1;
+          break;
+        }
+        r -= k.last;
+      }
     } else {
       for (j = 0;; ++j) {
-        const int e = esize(j + kAhead), o = nt - j - kEarly > 0 ? nt - j - kEarly : 0;
+        const int e = dag_early(nt, j + kAhead), o = nt - j - kEarly > 0 ? nt - j - kEarly : 0;
         if (r < e) {
           i = j + kAhead + r;
           j = j + kAhead;
@@ -1602,6 +1974,7 @@ __device__ __forceinline__ void dag_task(const DagArgs& g, int t, double* __rest
 // the workgroups to the XCDs in advance: when the only XCD with workgroups
 // left to start is full of waiting ones, the lowest untaken ticket never
 // starts.)
+template <bool MACRO>
 __global__ __launch_bounds__(256) void potrf_dag_kernel(DagArgs g) {
   // one LDS variable: with several, the compiler's record of which pointers
   // are distinct is lost, and LDS reads wait for every load into LDS before
@@ -1609,8 +1982,8 @@ __global__ __launch_bounds__(256) void potrf_dag_kernel(DagArgs g) {
   __shared__ __attribute__((aligned(16))) double smem[kDagSmemDoubles + 2];
   int& t_s = *reinterpret_cast<int*>(smem + kDagSmemDoubles);  // then the three words of pair_accumulate
   const int ns = g.s0 >= 0 ? g.nt - g.s0 : 0;
-  const int total = g.nt * (g.nt + 1) / 2 + ns * (ns + 1) / 2;  // the last ticket
-  for (;;) {
+  const int total = g.nfac + ns * (ns + 1) / 2;  // the last ticket
+  auto take = [&] {
     if (threadIdx.x == 0) {
       const int t = atomicAdd(&g.sync[0], 1);
       t_s = t;
@@ -1622,11 +1995,29 @@ __global__ __launch_bounds__(256) void potrf_dag_kernel(DagArgs g) {
     __syncthreads();
     const int t = __builtin_amdgcn_readfirstlane(t_s);
     __syncthreads();
-    if (t > total) break;
-    dag_task(g, t, smem);
+    return t;
+  };
+  int t = take();
+  // the walker outside the loop over tile tasks, so that what the compiler
+  // hoists out of either takes no registers from the other
+  if (t == 0) {
+    dag_walker(g, smem);
+    __syncthreads();
+    t = take();
+  }
+  for (; t <= total; t = take()) {
+    dag_task<MACRO>(g, t, smem);
     __syncthreads();
   }
 }
+
+// Block columns from which macro tasks take the place of the single tiles away
+// from the diagonal.  Below, a launch has too few of them to fill the CUs near
+// its end; single / macro ms for the 11N launch and the W_PP product after it:
+// N = 640 (110 block columns) 3.71 / 3.76, N = 720 (124) 5.15 / 5.27, N = 800
+// (138) 6.74 / 6.70, N = 900 (155) 9.57 / 9.33, N = 997 (172) 12.6 / 12.3,
+// N = 1400 (242) 35.9 / 33.0.
+constexpr int kMacroTiles = 136;
 
 // one persistent workgroup per CU
 static int dag_workgroups() {
@@ -1694,14 +2085,16 @@ int potrf_lower_x(DenseWork& w, double* A, int n, int ld, int s0, double* X, int
   const int rc = dag_reserve(w, nt, s);
   if (rc) return rc;
   if (++w.dag_gen == 0x7fffffff) w.dag_gen = 1;
-  DagArgs g{A, ld, nt, w.dinv, w.d_part, w.d_dag, w.dag_gen, w.d_info, w.d_rec, s0, X, ldx};
+  const bool macro = nt >= kMacroTiles;
+  const int nfac = dag_tickets(nt, macro);
+  DagArgs g{A, ld, nt, w.dinv, w.d_part, w.d_dag, w.dag_gen, nfac, w.d_info, w.d_rec, s0, X, ldx};
   const int ns = s0 >= 0 ? nt - s0 : 0;
   // algorithmic flops: n^3/3 for the factor, plus m^3/3 for the triangular inverse of its trailing
   // m = 64 ns rows when X is asked for
   const double nd = (double)n, md = 64.0 * ns;
   hipEvent_t pe = prof_begin(kProfPotrfDiag, (nd * nd * nd + md * md * md) / 3.0, 0.0, s);
-  hipLaunchKernelGGL(potrf_dag_kernel, dim3(std::min(1 + nt * (nt + 1) / 2 + ns * (ns + 1) / 2, dag_workgroups())),
-                     dim3(256), 0, s, g);
+  hipLaunchKernelGGL((macro ? potrf_dag_kernel<true> : potrf_dag_kernel<false>),
+                     dim3(std::min(1 + nfac + ns * (ns + 1) / 2, dag_workgroups())), dim3(256), 0, s, g);
   prof_end(pe, s);
   RSD_HIP(hipGetLastError());
   return RSD_OK;

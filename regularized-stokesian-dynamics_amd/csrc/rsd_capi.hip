@@ -1017,8 +1017,14 @@ extern "C" int rsd_ctx_create(rsd_ctx** out, int n, const rsd_step_config* cfg) 
   if (cfg->nb < 0 || cfg->nb > n || !(cfg->ews_err > 0.0) || !(cfg->mu_f > 0.0)) return RSD_ERR_ARG;
   std::unique_ptr<rsd_ctx> c(new rsd_ctx);
   RSD_HIP(hipGetDevice(&c->dev));
-  RSD_HIP(hipStreamCreateWithFlags(&c->s, hipStreamNonBlocking));
-  RSD_HIP(hipStreamCreateWithFlags(&c->s2, hipStreamNonBlocking));
+  // HIP deals streams out to its few hardware queues in the order of their
+  // creation: the order of the two changes every second context, so that the
+  // main streams of a batch take turns at all the queues and not at every other
+  // one (a batch of 12 at width 8: 59.6 -> 56.5 ms)
+  static std::atomic<unsigned> created{0};
+  const bool side_first = (created.fetch_add(1) >> 1) & 1;
+  RSD_HIP(hipStreamCreateWithFlags(side_first ? &c->s2 : &c->s, hipStreamNonBlocking));
+  RSD_HIP(hipStreamCreateWithFlags(side_first ? &c->s : &c->s2, hipStreamNonBlocking));
   RSD_HIP(hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming));
   RSD_HIP(hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming));
   RSD_HIP(hipEventCreateWithFlags(&c->ev_copied, hipEventDisableTiming));

@@ -2019,8 +2019,14 @@ __global__ __launch_bounds__(256) void potrf_dag_kernel(DagArgs g) {
 // N = 1400 (242) 35.9 / 33.0.
 constexpr int kMacroTiles = 136;
 
-// one persistent workgroup per CU
-static int dag_workgroups() {
+// The persistent workgroups of a launch of nt block columns: at most one per CU,
+// and no more than its tile work keeps busy beside the diagonal chain, so that
+// concurrent suspensions' factorisations share the chip (a workgroup takes all
+// of a CU's registers).  Fewest workgroups at which a launch alone is no
+// slower: 32 at 19 block columns, 64 at 32 and 35, 96 at 48, 160 at 58 and 60;
+// more than 160 at 88.  A batch of 12 suspensions of N = 108..640 takes 59.6 ms
+// so, and 64.2 with every launch on all CUs.
+static int dag_cus() {
   static int n = 0;
   if (n == 0) {
     int dev = 0, cus = 0;
@@ -2032,6 +2038,8 @@ static int dag_workgroups() {
   }
   return n;
 }
+
+static int dag_workgroups(int nt) { return std::min(dag_cus(), 16 + nt * nt / 24); }
 
 __global__ void dag_wait_reset_kernel(int* err, int* rec) {
   if (threadIdx.x == 0) *err = 0;
@@ -2094,7 +2102,7 @@ int potrf_lower_x(DenseWork& w, double* A, int n, int ld, int s0, double* X, int
   const double nd = (double)n, md = 64.0 * ns;
   hipEvent_t pe = prof_begin(kProfPotrfDiag, (nd * nd * nd + md * md * md) / 3.0, 0.0, s);
   hipLaunchKernelGGL((macro ? potrf_dag_kernel<true> : potrf_dag_kernel<false>),
-                     dim3(std::min(1 + nfac + ns * (ns + 1) / 2, dag_workgroups())), dim3(256), 0, s, g);
+                     dim3(std::min(1 + nfac + ns * (ns + 1) / 2, dag_workgroups(nt))), dim3(256), 0, s, g);
   prof_end(pe, s);
   RSD_HIP(hipGetLastError());
   return RSD_OK;

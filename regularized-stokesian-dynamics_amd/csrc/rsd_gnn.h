@@ -74,9 +74,7 @@ struct GnnWork {
   float* V = nullptr;      // edge pre-activations: 3 x N cap x 64
   float* OUT = nullptr;    // the pair weight's logit per slot
   float* dOUT = nullptr;
-  float* dH = nullptr;     // 3 x N x 64 (two ping-pong + a partial)
-  float* dU = nullptr;     // N x 64
-  float* dV = nullptr;     // N cap x 64
+  float* bwd = nullptr;    // the backward pass's sums per particle (GnnBwd)
   float* grad = nullptr;   // kGnnParams
   float* gpart = nullptr;  // split reductions
   double* zv = nullptr;    // nz Gaussian vectors (11N each)

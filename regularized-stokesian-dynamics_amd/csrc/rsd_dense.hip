@@ -556,64 +556,69 @@ __device__ __forceinline__ double rsqrt_nr(double d) {
   return fma(y0 * e, fma(0.375, e, 0.5), y0);
 }
 
-// Wave-uniform read of a double held by one lane (lane index known at
-// compile time in the unrolled pivot loop).
-__device__ __forceinline__ double readlane_d(double v, int lane) {
-  const long long u = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_readlane((int)u, lane);
-  const int hi = __builtin_amdgcn_readlane((int)(u >> 32), lane);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+// lane N of each row of 16 lanes to the whole row
+template <int N>
+__device__ __forceinline__ double row_bcast(double v) {
+  return __builtin_amdgcn_update_dpp(v, v, 0x150 + N, 0xf, 0xf, true);
 }
 
-// D += P(16x16) * Q(16x16) on the matrix cores; P and Q point at the
-// blocks' first elements in row-major LDS arrays with row strides PS, QS.
-template <int PS, int QS>
-__device__ __forceinline__ v4d mm16(const double* P, const double* Q, v4d acc, int lane) {
-  const int r = lane & 15, kq = lane >> 4;
+// D += P(16x16) * Q(16x16) on the matrix cores: P points at the block's first
+// element in a row-major LDS array with row stride PS, Q is in registers in the
+// layout of a result (lane: rows (lane>>4)+4v of column lane&15), which is also
+// that of the right operand's k-steps v and, for Q^T, of the left operand's: a
+// product's result feeds the next one without a trip through LDS.
+template <int PS>
+__device__ __forceinline__ v4d mm16(const double* P, const v4d& q, v4d acc, int lane) {
+  double a[4];
 #pragma unroll
-  for (int kb = 0; kb < 4; ++kb)
-    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(P[r * PS + 4 * kb + kq], Q[(4 * kb + kq) * QS + r], acc, 0, 0, 0);
+  for (int kb = 0; kb < 4; ++kb) a[kb] = P[(lane & 15) * PS + 4 * kb + (lane >> 4)];
+#pragma unroll
+  for (int kb = 0; kb < 4; ++kb) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[kb], q[kb], acc, 0, 0, 0);
   return acc;
 }
 
 struct DiagSmem {
-  double col[16][64];    // the owner wave's scaled columns, for its own deferred updates
-  double P[2][64][18];   // finished 16-column panels, for the waves to their right
-  double Ls[64][65];     // the factor, written panel by panel (upper triangle zero)
+  double P[4][64][18];   // the factor by 16-column panels, rows below the panel's diagonal block
   double Xs[64][65];     // its inverse, lower 16x16 blocks
-  double Tt[8][16][17];  // partial sums of the inverse's off-diagonal blocks
-  double U[48][66];      // the previous panel's rank-16 term for columns 16..63, [column - 16][row]
-  double ry[64];         // 1 / L_jj: the pivots' reciprocal square roots
+  double R[64][65];      // the tile; then U, the previous panel's rank-16 term: [column - 16][row], rows of 66
+  double T[64][66];      // the next column's tile (j+1,j) of the factor, transposed
   int bad;
+  int ready;             // 1 + the last column whose partial tiles are known to be published
+  int stored;            // waves whose part of an inverse is stored, over all columns
 };
 
-// X_bb = inv(L_bb) for diagonal block b, by one wave: lane c < 16 solves
-// column c by column-oriented forward substitution (16 steps on the chain,
-// the row updates of a step independent of one another), with the pivots'
-// reciprocals from the factorization instead of divides.  (Reading L_bb's
-// columns ahead into registers is faster alone, but the walker is at its
-// register limit here and then spills.)
-__device__ __forceinline__ void diag_block_inverse(DiagSmem& sm, int b, int l) {
-  if (l < 16) {
-    double x[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) x[i] = (i == l) ? 1.0 : 0.0;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      x[k] *= sm.ry[16 * b + k];
-#pragma unroll
-      for (int i = k + 1; i < 16; ++i) x[i] -= sm.Ls[16 * b + i][16 * b + k] * x[k];
-    }
-#pragma unroll
-    for (int i = 0; i < 16; ++i) sm.Xs[16 * b + i][16 * b + l] = x[i];
+// columns Q2 .. 15 less a pivot's term
+template <int Q2>
+__device__ __forceinline__ void panel_terms(double (&dg)[16], double (&a)[16], double vd, double va) {
+  if constexpr (Q2 < 16) {
+    const double m = row_bcast<Q2>(vd);
+    dg[Q2] = fma(-vd, m, dg[Q2]);
+    a[Q2] = fma(-va, m, a[Q2]);
+    panel_terms<Q2 + 1>(dg, a, vd, va);
   }
+}
+// Pivots Q .. 15 of a 16x16 block and its share of the rows below.  Each of the
+// four rows of 16 lanes holds the block, lane i its row i in dg, so that every
+// multiplier is a broadcast within 16 lanes (one instruction); a is one more
+// row per lane, solved along.  A bit of `ok` per positive pivot.
+template <int Q>
+__device__ __forceinline__ void panel_pivots(double (&dg)[16], double (&a)[16], unsigned& ok) {
+  const double d = row_bcast<Q>(dg[Q]);
+  const double y = rsqrt_nr(d);
+  ok |= ((unsigned)__ballot(d > 0.0) & 1u) << Q;
+  const double vd = dg[Q] * y, va = a[Q] * y;
+  dg[Q] = vd;
+  a[Q] = va;
+  panel_terms<Q + 1>(dg, a, vd, va);
+  if constexpr (Q + 1 < 16) panel_pivots<Q + 1>(dg, a, ok);
 }
 
 // 16x16 blocks in MFMA layout (lane holds rows (lane>>4)+4v of column lane&15)
-__device__ __forceinline__ v4d blk_load(const double (*T)[17], int lane) {
+template <int DS>
+__device__ __forceinline__ v4d blk_load(const double* src, int lane) {
   v4d t;
 #pragma unroll
-  for (int v = 0; v < 4; ++v) t[v] = T[(lane >> 4) + 4 * v][lane & 15];
+  for (int v = 0; v < 4; ++v) t[v] = src[((lane >> 4) + 4 * v) * DS + (lane & 15)];
   return t;
 }
 template <int DS>
@@ -621,69 +626,57 @@ __device__ __forceinline__ void blk_store(double* dst, v4d t, double sign, int l
 #pragma unroll
   for (int v = 0; v < 4; ++v) dst[((lane >> 4) + 4 * v) * DS + (lane & 15)] = sign * t[v];
 }
-// a volatile int in LDS, addressed as such (a generic pointer would make the
-// access a flat one, which also waits on the vector memory counter)
-__device__ __forceinline__ volatile __attribute__((address_space(3))) int* lds_int(int* p) {
-  return (volatile __attribute__((address_space(3))) int*)(p);
-}
-__device__ __forceinline__ volatile __attribute__((address_space(3))) double* lds_dbl(double* p) {
-  return (volatile __attribute__((address_space(3))) double*)(p);
-}
-// a NaN with a payload no arithmetic produces: "not written yet"
-constexpr double kNotYet = __builtin_bit_cast(double, 0x7ff4dead0000beefull);
-__device__ __forceinline__ bool not_yet(double v) {
-  return __double_as_longlong(v) == 0x7ff4dead0000beefll;
-}
-// 1/d to full FP64 accuracy: the hardware estimate and two Newton steps
-__device__ __forceinline__ double recip(double d) {
-  double r = __builtin_amdgcn_rcp(d);
-  r = fma(fma(-d, r, 1.0), r, r);
-  return fma(fma(-d, r, 1.0), r, r);
-}
 // orders a wave's LDS writes before its later reads of other lanes' elements
 __device__ __forceinline__ void wave_lds_order() { __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront"); }
 
 // Cholesky of one 64x64 diagonal tile held in registers by 256 threads, and
 // its triangular inverse: thread (w, l) has row l, columns 16w..16w+15 in
-// a[].  The tile is done in four 16-column panels.  The wave that owns a
-// panel factors it alone, as a software pipeline around the serial pivot
-// chain (lane read of the pivot, rsqrt_nr, scale, lane read of the next
-// column's entry): every other update of pivot q uses column entries read
-// from LDS one iteration earlier.  The finished panel goes to LDS; after a
-// barrier, its rank-16 term for all the columns to its right is formed by
-// MFMA 16x16x16 products (the lower blocks only, spread over the waves) and
-// handed over through LDS after a second barrier: each wave subtracts its
-// own columns' term, and the owner's pivot loop carries no term of the
-// previous panel.
-// The inverse X = inv(L) is built from 16x16 blocks, X_bb = inv(L_bb) and
-// X_bm = -X_bb (sum_{m'=m}^{b-1} L_bm' X_m'm), on the waves that the panels
-// leave idle: the blocks of panels 0..2 while the later panels factor, and
-// after the last panel two levels of MFMA 16x16x16 products over all four
-// waves.
-// On return (after a barrier) sm.Ls holds L (upper triangle zero), sm.Xs the
-// lower blocks of X, and sm.bad the LAPACK-style INFO of the first
-// non-positive pivot (k0 + j + 1) or 0x7fffffff.
-// hook(b) runs while panel b+1 is factored (b = 0..2) on the waves that do
-// not own it, and after the first level of the last products on every
-// wave: points where a wave has slack.
-template <class Hook>
-__device__ __forceinline__ void diag_factor64(double (&a)[16], DiagSmem& sm, int k0, Hook&& hook) {
-  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63;
-  if (tid == 0) sm.bad = 0x7fffffff;
+// a[], and row 16w + l%16 of the same columns in dg[].  The tile is done in
+// four 16-column panels, panel b by wave b alone: the pivot chain runs on its
+// diagonal block, which each row of 16 lanes holds for itself (panel_pivots),
+// and lane l's row of the panel follows it.  The lanes of the diagonal block's
+// own rows solve the identity's rows instead, which gives X_bb^T = L_bb^-T
+// with the panel.  A pivot is bound by its chain, broadcast, reciprocal square
+// root, scale, next column's term, with the other columns' terms between.
+// The finished panel goes to LDS; after a barrier, its rank-16 term for all
+// the columns to its right is formed by MFMA 16x16x16 products (the lower
+// blocks only, spread over the waves) and handed over through LDS after a
+// second barrier.
+// The inverse's other blocks: wave m < 3 has column m, X_im = -X_ii sum_{k=m}^{i-1}
+// L_ik X_km, the sums and blocks in registers; a sum grows by one product per
+// panel while the wave has no panel of its own, and after the last one only
+// the products with X_33 are left.
+// A 64x64 tile and its inverse take 21k clocks so (a panel's 16 pivots 2.4k); with
+// the multipliers read from lanes and LDS, X_bb by substitutions of their own and
+// two levels of products after the last panel they took 34.5k.
+// On return sm.P holds L's panels, sm.Xs the lower blocks of X, sm.bad the
+// LAPACK-style INFO of the first non-positive pivot (k0 + j + 1) or 0x7fffffff,
+// a[] this wave's columns of L in the rows below the diagonal block and dg[]
+// the block's own rows; a barrier has to follow.
+// idle(b) runs while panel b is factored on the waves that do not own it, last()
+// on all when the panels are done, before the last products.
+template <class Idle, class Last>
+__device__ __forceinline__ void diag_factor64(double (&a)[16], double (&dg)[16], DiagSmem& sm, int k0, Idle&& idle,
+                                              Last&& last) {
+  const int w = __builtin_amdgcn_readfirstlane(opaque_tid() >> 6);
+  if (threadIdx.x == 0) sm.bad = 0x7fffffff;
   const v4d z = {0.0, 0.0, 0.0, 0.0};
-  auto Lb = [&](int i, int m) { return &sm.Ls[16 * i][16 * m]; };
-  auto Xb = [&](int i, int m) { return &sm.Xs[16 * i][16 * m]; };
-  auto Tb = [&](int s) { return &sm.Tt[s][0][0]; };
-#pragma unroll
+  double(*U)[66] = reinterpret_cast<double(*)[66]>(&sm.R[0][0]);
+  v4d xt[4] = {z, z, z, z};  // the sums for X_im, i > m = w
+#pragma unroll 1
   for (int b = 0; b < 4; ++b) {
-    double(*P)[18] = sm.P[b & 1];
-    double(*Pp)[18] = sm.P[(b + 1) & 1];  // the previous panel (b-1)
+    const int l = opaque_tid() & 63;  // (LDS addresses not kept over the panels: there are too many)
     if (b > 0) {
       // U = the previous panel's rank-16 term for the columns to its right:
       // block (rb, cb) = Pp[16rb.., :] Pp[16cb.., :]^T for rb >= cb >= b (the
       // blocks above the diagonal are not needed), by MFMA, spread over the
       // waves; every wave then subtracts its own columns' blocks
-      auto u_block = [&](int rb, int cb) {
+      double(*Pp)[18] = sm.P[b - 1];
+      for (int n = w; n < (4 - b) * (5 - b) / 2; n += 4) {
+        // block n, by columns
+        int cb = b, k = n;
+        while (k >= 4 - cb) k -= 4 - cb++;
+        const int rb = cb + k;
         const int r = l & 15, kq = l >> 4;
         v4d u = z;
 #pragma unroll
@@ -691,192 +684,79 @@ __device__ __forceinline__ void diag_factor64(double (&a)[16], DiagSmem& sm, int
           u = __builtin_amdgcn_mfma_f64_16x16x4f64(Pp[16 * rb + r][4 * kb + kq], Pp[16 * cb + r][4 * kb + kq], u, 0,
                                                    0, 0);
 #pragma unroll
-        for (int v = 0; v < 4; ++v) sm.U[16 * (cb - 1) + r][16 * rb + kq + 4 * v] = u[v];
-      };
-      if (b == 1) {
-        if (w == 0) { u_block(1, 1); u_block(3, 3); }
-        if (w == 1) { u_block(2, 1); u_block(2, 2); }
-        if (w == 2) u_block(3, 1);
-        if (w == 3) u_block(3, 2);
-      }
-      if (b == 2) {
-        if (w == 0) u_block(2, 2);
-        if (w == 1) u_block(3, 2);
-        if (w == 2) u_block(3, 3);
-      }
-      if (b == 3 && w == 0) u_block(3, 3);
-      if (b == 3 && w == 1) {
-        // the last panel's columns, rows 48..63, marked as not yet written
-        // (the wave that inverts L_33 behind the pivots watches them)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) sm.col[4 * (l >> 4) + r][48 + (l & 15)] = kNotYet;
+        for (int v = 0; v < 4; ++v) U[16 * (cb - 1) + r][16 * rb + kq + 4 * v] = u[v];
       }
       __syncthreads();
       if (w >= b) {
-        // rows above the column block are above the diagonal: not needed
+        // (rows above the column block are above the diagonal: a is not read there)
+        const double *ud = &U[16 * (w - 1)][16 * w + (l & 15)], *ua = &U[16 * (w - 1)][l];
+        double td[16], ta[16];  // (all read, then subtracted: left to itself the compiler waits for each pair)
 #pragma unroll
-        for (int q = 0; q < 16; ++q) a[q] -= sm.U[16 * (w - 1) + q][l];
-      }
-      // the inverse's blocks that panels 0..b-1 allow, on the waves left of
-      // this panel's owner (Tt slots: 0 L10 X00, 1 L21 X11, 2 L20 X00,
-      // 3 L31 X11, 4 L30 X00)
-      if (b == 1 && w == 0) diag_block_inverse(sm, 0, l);
-      if (b == 2) {
-        if (w == 1) diag_block_inverse(sm, 1, l);
-        if (w == 0) blk_store<17>(Tb(0), mm16<65, 65>(Lb(1, 0), Xb(0, 0), z, l), 1.0, l);
-      }
-      if (b == 3) {
-        if (w == 2) diag_block_inverse(sm, 2, l);
-        if (w == 1) {
-          blk_store<65>(Xb(1, 0), mm16<65, 17>(Xb(1, 1), Tb(0), z, l), -1.0, l);
-          blk_store<17>(Tb(1), mm16<65, 65>(Lb(2, 1), Xb(1, 1), z, l), 1.0, l);
-        }
-        if (w == 0) {
-          blk_store<17>(Tb(2), mm16<65, 65>(Lb(2, 0), Xb(0, 0), z, l), 1.0, l);
-          blk_store<17>(Tb(3), mm16<65, 65>(Lb(3, 1), Xb(1, 1), z, l), 1.0, l);
-          blk_store<17>(Tb(4), mm16<65, 65>(Lb(3, 0), Xb(0, 0), z, l), 1.0, l);
-        }
-      }
-      if (w != b) hook(b - 1);
-      if (b == 3 && w == 1) {
-        // X_33 = inv(L_33) behind the last panel's pivots, by column-oriented
-        // substitution as in diag_block_inverse, so that it is done when the
-        // panel is.  Step k waits until column k's entries in rows 48..63 are
-        // no longer marked (the owner writes a column with one LDS store),
-        // and forms 1/L_kk itself.  Lane (g, c) holds rows 4g..4g+3 of column
-        // c (few registers: the walker is near its limit here); step k's x_k
-        // comes from lane (k/4, c) by a shuffle.
-        const int c = l & 15, g = l >> 4;
-        double x[4], d, e[4];
+        for (int q = 0; q < 16; ++q) td[q] = ud[66 * q], ta[q] = ua[66 * q];
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) x[r] = (4 * g + r == c) ? 1.0 : 0.0;
-        // column k's diagonal entry and this lane's four entries, once written
-        auto fetch = [&](int k) {
-          bool pending;
-          do {
-            d = *lds_dbl(&sm.col[k][48 + k]);
-            pending = not_yet(d);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              e[r] = *lds_dbl(&sm.col[k][48 + 4 * g + r]);
-              pending |= not_yet(e[r]);
-            }
-            if (pending) __builtin_amdgcn_s_sleep(1);
-          } while (pending);
-        };
-        fetch(0);
-        double rk = recip(d);
-        // step k; column k+1 is fetched and its reciprocal formed while step
-        // k's shuffle is in flight
-#pragma unroll
-        for (int k = 0; k < 16; ++k) {
-          const double xs = x[k & 3] * rk;
-          if (g == (k >> 2)) x[k & 3] = xs;
-          const double xk = __shfl(xs, 16 * (k >> 2) + c, 64);
-          double ek[4];
-#pragma unroll
-          for (int r = 0; r < 4; ++r) ek[r] = e[r];
-          if (k + 1 < 16) {
-            fetch(k + 1);
-            rk = recip(d);
-          }
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-            if (4 * g + r > k) x[r] -= ek[r] * xk;
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) sm.Xs[48 + 4 * g + r][48 + c] = x[r];
+        for (int q = 0; q < 16; ++q) dg[q] -= td[q], a[q] -= ta[q];
       }
     }
     if (w == b) {
-      int first_bad = 64;
-      double yq = 0.0, vprev = 0.0, rd[16];
+      const int g = l >> 4, i = l & 15;
+      unsigned ok = 0;
+      if (g == b) {
 #pragma unroll
-      for (int q = 0; q < 16; ++q) rd[q] = 0.0;
-#pragma unroll
-      for (int q = 0; q < 16; ++q) {
-        const int j = 16 * b + q;
-        const double dj = readlane_d(a[q], j);
-        first_bad = (dj > 0.0 || first_bad < 64) ? first_bad : j;
-        const double y = rsqrt_nr(dj);
-        yq = (l == q) ? y : yq;
-        // lane j holds dj itself, so one product gives both L_jj and the column
-        const double v = (l >= j) ? a[q] * y : 0.0;
-        a[q] = v;
-        sm.col[q][l] = v;
-        if (q + 1 < 16) {
-          // column q+1 before the next pivot: the previous pivot's term
-          // (operands already in registers), then this pivot's term by a lane
-          // read (the serial chain)
-          if (q >= 1) a[q + 1] -= vprev * rd[q + 1];
-          a[q + 1] -= v * readlane_d(v, j + 1);
-        }
-        // the previous pivot's terms for the columns right of q+1, from registers
-        if (q >= 1) {
-#pragma unroll
-          for (int q2 = q + 2; q2 < 16; ++q2) a[q2] -= vprev * rd[q2];
-        }
-        // this pivot's column entries, read now and used one iteration later
-#pragma unroll
-        for (int q2 = q + 2; q2 < 16; ++q2) rd[q2] = sm.col[q][16 * b + q2];
-        vprev = v;
+        for (int q = 0; q < 16; ++q) a[q] = (q == i) ? 1.0 : 0.0;
       }
+      panel_pivots<0>(dg, a, ok);
+      if (g == b) {
+        // a is row i of X_bb^T, dg row i of L_bb
 #pragma unroll
-      for (int q = 0; q < 16; ++q) P[l][q] = a[q];
+        for (int q = 0; q < 16; ++q) sm.Xs[16 * b + q][l] = a[q];
+      }
+      // (nothing reads the rows of the diagonal block or above it)
 #pragma unroll
-      for (int q = 0; q < 16; ++q) sm.Ls[l][16 * b + q] = a[q];
-      if (l < 16) sm.ry[16 * b + l] = yq;
-      if (first_bad < 64 && l == 0) atomicMin(&sm.bad, k0 + first_bad + 1);
+      for (int q = 0; q < 16; ++q) sm.P[b][l][q] = a[q];
+      if (ok != 0xffffu && l == 0) atomicMin(&sm.bad, k0 + 16 * b + __builtin_ctz(~ok) + 1);
+    } else {
+      if (w < b && w < 3) {
+        // X_{b-1,w}, and its products for the sums of the rows below
+        const int k = b - 1;
+        v4d x;
+        if (k == w) {
+          x = blk_load<65>(&sm.Xs[16 * w][16 * w], l);
+        } else {
+          const v4d t = k == 1 ? xt[1] : xt[2];
+          x = -mm16<65>(&sm.Xs[16 * k][16 * k], t, z, l);
+          blk_store<65>(&sm.Xs[16 * k][16 * w], x, 1.0, l);
+        }
+#pragma unroll
+        for (int i = 1; i < 4; ++i)
+          if (i >= b) xt[i] = mm16<18>(&sm.P[k][16 * i][0], x, xt[i], l);
+      }
+      idle(b);
     }
     __syncthreads();
   }
-  // after the last panel (X_33 is done by then): X_21, X_20, then X_32, X_31, X_30
-  // (Tt slots: 5 L20 X00 + L21 X10, 6 L32 X22, 7 L30 X00 + L31 X10)
-  if (w == 2) blk_store<65>(Xb(2, 1), mm16<65, 17>(Xb(2, 2), Tb(1), z, l), -1.0, l);
-  if (w == 1) {
-    blk_store<17>(Tb(5), mm16<65, 65>(Lb(2, 1), Xb(1, 0), blk_load(sm.Tt[2], l), l), 1.0, l);
-    wave_lds_order();
-    blk_store<65>(Xb(2, 0), mm16<65, 17>(Xb(2, 2), Tb(5), z, l), -1.0, l);
+  // the inverse's last row of blocks
+  last();
+  if (w < 3) {
+    const int l = opaque_tid() & 63;
+    blk_store<65>(&sm.Xs[48][16 * w], mm16<65>(&sm.Xs[48][48], xt[3], z, l), -1.0, l);
   }
-  if (w == 0) {
-    blk_store<17>(Tb(6), mm16<65, 65>(Lb(3, 2), Xb(2, 2), z, l), 1.0, l);
-    blk_store<17>(Tb(7), mm16<65, 65>(Lb(3, 1), Xb(1, 0), blk_load(sm.Tt[4], l), l), 1.0, l);
-  }
-  hook(3);
-  __syncthreads();
-  if (w == 0) blk_store<65>(Xb(3, 2), mm16<65, 17>(Xb(3, 3), Tb(6), z, l), -1.0, l);
-  if (w == 1) {
-    blk_store<17>(Tb(3), mm16<65, 65>(Lb(3, 2), Xb(2, 1), blk_load(sm.Tt[3], l), l), 1.0, l);
-    wave_lds_order();
-    blk_store<65>(Xb(3, 1), mm16<65, 17>(Xb(3, 3), Tb(3), z, l), -1.0, l);
-  }
-  if (w == 2) {
-    blk_store<17>(Tb(7), mm16<65, 65>(Lb(3, 2), Xb(2, 0), blk_load(sm.Tt[7], l), l), 1.0, l);
-    wave_lds_order();
-    blk_store<65>(Xb(3, 0), mm16<65, 17>(Xb(3, 3), Tb(7), z, l), -1.0, l);
-  }
-  __syncthreads();
 }
 
-// the inverse (column-major, zero upper blocks; written through) and the INFO word
-__device__ __forceinline__ void diag_store_inverse(const DiagSmem& sm, double* __restrict__ dinv, int* __restrict__ info) {
-  const int tid = opaque_tid(), w = tid >> 6, l = tid & 63;
+// the factor (this wave's columns in a and dg, as diag_factor64 leaves them)
+// into the matrix, from its element (k0, k0) at A
+__device__ __forceinline__ void diag_store_factor(const double (&a)[16], const double (&dg)[16],
+                                                  double* __restrict__ A, size_t ld) {
+  const int tid = opaque_tid(), w = tid >> 6, l = tid & 63, g = l >> 4, i = l & 15;
 #pragma unroll
-  for (int q = 0; q < 16; ++q) {
-    const int c = 16 * w + q;
-    wt_store(dinv + (size_t)l + (size_t)c * 64, ((l >> 4) >= w) ? sm.Xs[l][c] : 0.0);
-  }
-  if (tid == 0 && sm.bad != 0x7fffffff) atomicMin(info, sm.bad);
+  for (int q = 0; q < 16; ++q)
+    A[(size_t)l + (size_t)(16 * w + q) * ld] = g > w ? a[q] : (g == w && q <= i) ? dg[q] : 0.0;
 }
-
-// the factor into the matrix at (k0, k0)
-__device__ __forceinline__ void diag_store_factor(const DiagSmem& sm, double* __restrict__ A, int ld, int k0) {
-  const int tid = opaque_tid(), w = tid >> 6, l = tid & 63;
-#pragma unroll
-  for (int q = 0; q < 16; ++q) {
-    const int c = 16 * w + q;
-    A[(size_t)(k0 + l) + (size_t)(k0 + c) * ld] = sm.Ls[l][c];
-  }
+// rows 16 rb .. of the inverse, columns 4n .. 4n+3 (column-major, zero upper
+// blocks; written through)
+__device__ __forceinline__ void diag_store_inverse(const DiagSmem& sm, double* __restrict__ dinv, int rb, int n, int lane) {
+  const int r = 16 * rb + (lane & 15), c = 4 * n + (lane >> 4);
+  wt_store(dinv + r + (size_t)c * 64, n < 4 * rb + 4 ? sm.Xs[r][c] : 0.0);
 }
 
 __global__ void set_int_kernel(int* p, int v) { *p = v; }
@@ -931,11 +811,11 @@ __device__ __forceinline__ void wait_flag(const int* flag, int gen, int* err, in
 // Ticket 0 is the walker: one workgroup that runs the serial chain down the
 // diagonal by itself.  For column j it takes the partial sum of tile (j,j)
 // (all updates but the last), subtracts the last update L_{j,j-1} L_{j,j-1}^T
-// from the tile it computed one column earlier and still holds in
-// registers, factors the tile (diag_factor64, which also writes the 64x64
-// inverse), publishes it, and then turns the partial sum of tile (j+1,j)
-// into L_{j+1,j} with the inverse it has just built.  No hand-off between
-// workgroups sits on the diagonal chain.
+// from the tile it computed one column earlier and still has in LDS,
+// factors the tile (diag_factor64, which also forms the 64x64 inverse),
+// publishes the inverse, and turns the partial sum of tile (j+1,j) into
+// L_{j+1,j} by forward substitution with the factor's 16x16 blocks.  No
+// hand-off between workgroups sits on the diagonal chain.
 //
 // Tickets 1.. are the lower tiles (i,j), one workgroup each: first the
 // early tiles (c,c), (c+1,c), (c+2,c) of columns 0..kAhead-1, then for each
@@ -973,7 +853,7 @@ struct DagArgs {
   double* A;
   int ld, nt;
   double* dinv;  // nt inverted 64x64 diagonal factors, column-major
-  double* part;  // 2 nt partial tiles, column-major 64x64: (j,j) at 2j, (j+1,j) at 2j+1;
+  double* part;  // 2 nt partial tiles (part_at): (j,j) at 2j, (j+1,j), transposed, at 2j+1;
                  // then (with X) the transposed diagonal blocks of X, ns tiles
   int* sync;     // [0] ticket, [1] error word, [2, 2+nt*nt) tile flags, then 2 nt partial
                  // flags, then (with X) ns*ns flags of X's tiles
@@ -1006,20 +886,14 @@ __device__ __forceinline__ void tile_load(v4d (&acc)[2][2], const double* src, s
       }
 }
 
-// a published 64x64 tile (column-major, leading dimension 64) as the A
-// operands of a 64-deep MFMA product: a0[st] = P(wm + m, 4 st + kq),
-// a1[st] = P(wm + 16 + m, 4 st + kq), m = lane & 15, kq = lane >> 4
-__device__ __forceinline__ void tile_load_a(double (&a0)[16], double (&a1)[16], const double* src) {
-  const int tid = opaque_tid(), lane = tid & 63, wave = tid >> 6;
-  const int wm = (wave & 1) * 32, m = lane & 15, kq = lane >> 4;
-#pragma unroll
-  for (int st = 0; st < 16; ++st) {
-    a0[st] = wt_load(src + (wm + m) + (4 * st + kq) * 64);
-    a1[st] = wt_load(src + (wm + 16 + m) + (4 * st + kq) * 64);
-  }
+// The columns of a solved tile in registers: waves 0, 1 have the 16-column
+// blocks 0 and 3, waves 2, 3 the blocks 1 and 2 (elsewhere 0, 1 and 2, 3).
+template <bool SOLVED>
+__device__ __forceinline__ int tile_col(int wave, int bn) {
+  return 16 * (SOLVED ? (bn ? 3 - (wave >> 1) : wave >> 1) : 2 * (wave >> 1) + bn);
 }
-
-__device__ __forceinline__ void tile_store_direct(const v4d (&acc)[2][2], double* dst, size_t ld) {
+// the transpose of a 64x64 tile into accumulator layout
+__device__ __forceinline__ void tile_load_t(v4d (&acc)[2][2], const double* src, size_t ld) {
   const int tid = opaque_tid(), lane = tid & 63, wave = tid >> 6;
   const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
 #pragma unroll
@@ -1028,21 +902,50 @@ __device__ __forceinline__ void tile_store_direct(const v4d (&acc)[2][2], double
     for (int bn = 0; bn < 2; ++bn)
 #pragma unroll
       for (int v = 0; v < 4; ++v)
-        wt_store(dst + (size_t)(wm + 16 * bm + (lane >> 4) + 4 * v) + (size_t)(wn + 16 * bn + (lane & 15)) * ld,
+        acc[bm][bn][v] = src[(size_t)(wn + 16 * bn + (lane & 15)) + (size_t)(wm + 16 * bm + (lane >> 4) + 4 * v) * ld];
+}
+// The walker's partial tiles are kept as it loads them: 16x16 block (rb, cb) in
+// MFMA layout, register v of the lanes in lane order at part_at(rb, cb, v), so
+// that a store or load is 512 bytes in a row (as a matrix, 16 pieces of 32: the
+// stores of a tile then took 2.3 us, on the chain).
+__device__ __forceinline__ int part_at(int rb, int cb, int v) { return ((4 * rb + cb) * 4 + v) * 64; }
+__device__ __forceinline__ void part_store(const v4d (&acc)[2][2], double* dst) {
+  const int tid = opaque_tid(), lane = tid & 63, wave = tid >> 6;
+#pragma unroll
+  for (int bm = 0; bm < 2; ++bm)
+#pragma unroll
+    for (int bn = 0; bn < 2; ++bn)
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+        wt_store(dst + part_at(2 * (wave & 1) + bm, 2 * (wave >> 1) + bn, v) + lane, acc[bm][bn][v]);
+}
+
+template <bool SOLVED>
+__device__ __forceinline__ void tile_store_direct(const v4d (&acc)[2][2], double* dst, size_t ld) {
+  const int tid = opaque_tid(), lane = tid & 63, wave = tid >> 6;
+  const int wm = (wave & 1) * 32;
+#pragma unroll
+  for (int bm = 0; bm < 2; ++bm)
+#pragma unroll
+    for (int bn = 0; bn < 2; ++bn)
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+        wt_store(dst + (size_t)(wm + 16 * bm + (lane >> 4) + 4 * v) + (size_t)(tile_col<SOLVED>(wave, bn) + (lane & 15)) * ld,
                  acc[bm][bn][v]);
 }
 
 // the transpose of a tile held in accumulator layout, written through
+template <bool SOLVED>
 __device__ __forceinline__ void tile_store_direct_t(const v4d (&acc)[2][2], double* dst, size_t ld) {
   const int tid = opaque_tid(), lane = tid & 63, wave = tid >> 6;
-  const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
+  const int wm = (wave & 1) * 32;
 #pragma unroll
   for (int bm = 0; bm < 2; ++bm)
 #pragma unroll
     for (int bn = 0; bn < 2; ++bn)
 #pragma unroll
       for (int v = 0; v < 4; ++v)
-        wt_store(dst + (size_t)(wn + 16 * bn + (lane & 15)) + (size_t)(wm + 16 * bm + (lane >> 4) + 4 * v) * ld,
+        wt_store(dst + (size_t)(tile_col<SOLVED>(wave, bn) + (lane & 15)) + (size_t)(wm + 16 * bm + (lane >> 4) + 4 * v) * ld,
                  acc[bm][bn][v]);
 }
 
@@ -1586,7 +1489,32 @@ static int dag_tickets(int nt, bool macro) {
   return n;
 }
 
-// out = acc Dinv^T, Dinv a column-major 64x64 tile in global memory
+// Column blocks C0 < C1 of out = C Dinv^T for this wave's 32 rows: Dinv^T is zero
+// below its block diagonal, so block c takes the k-steps 0 .. 4c+3 only, 40
+// products a wave instead of 64.
+template <int C0, int C1>
+__device__ __forceinline__ void trsm_product(v4d (&out)[2][2], const double (*Cs)[66], const double* Dj, int wm, int lane) {
+  constexpr int S0 = 4 * (C0 + 1), S1 = 4 * (C1 + 1);
+  double a0[S1], a1[S1], b0[S0], b1[S1];  // every step's operands read ahead of the MFMAs
+#pragma unroll
+  for (int st = 0; st < S1; ++st) {
+    const int kr = 4 * st + (lane >> 4);
+    a0[st] = Cs[kr][wm + (lane & 15)];
+    a1[st] = Cs[kr][wm + 16 + (lane & 15)];
+    if (st < S0) b0[st < S0 ? st : 0] = Dj[staged(16 * C0 + (lane & 15), kr)];
+    b1[st] = Dj[staged(16 * C1 + (lane & 15), kr)];
+  }
+#pragma unroll
+  for (int st = 0; st < S1; ++st) {
+    if (st < S0) {
+      out[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0[st], b0[st < S0 ? st : 0], out[0][0], 0, 0, 0);
+      out[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1[st], b0[st < S0 ? st : 0], out[1][0], 0, 0, 0);
+    }
+    out[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0[st], b1[st], out[0][1], 0, 0, 0);
+    out[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1[st], b1[st], out[1][1], 0, 0, 0);
+  }
+}
+// out = acc Dinv^T, Dinv a column-major lower triangular 64x64 tile in global memory (out's columns: tile_col<true>)
 __device__ __forceinline__ void tile_trsm(const v4d (&acc)[2][2], const double* __restrict__ Dg, double* smem,
                                           v4d (&out)[2][2]) {
   const int tid = opaque_tid(), lane = tid & 63, wave = tid >> 6;
@@ -1607,22 +1535,8 @@ __device__ __forceinline__ void tile_trsm(const v4d (&acc)[2][2], const double* 
   for (int bm = 0; bm < 2; ++bm)
 #pragma unroll
     for (int bn = 0; bn < 2; ++bn) out[bm][bn] = (v4d){0.0, 0.0, 0.0, 0.0};
-  double a0[16], a1[16], b0[16], b1[16];  // every step's operands read ahead of the MFMAs
-#pragma unroll
-  for (int st = 0; st < 16; ++st) {
-    const int kr = 4 * st + (lane >> 4);
-    a0[st] = Cs[kr][wm + (lane & 15)];
-    a1[st] = Cs[kr][wm + 16 + (lane & 15)];
-    b0[st] = Dj[staged(wn + (lane & 15), kr)];
-    b1[st] = Dj[staged(wn + 16 + (lane & 15), kr)];
-  }
-#pragma unroll
-  for (int st = 0; st < 16; ++st) {
-    out[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0[st], b0[st], out[0][0], 0, 0, 0);
-    out[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0[st], b1[st], out[0][1], 0, 0, 0);
-    out[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1[st], b0[st], out[1][0], 0, 0, 0);
-    out[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1[st], b1[st], out[1][1], 0, 0, 0);
-  }
+  if (wave >> 1) trsm_product<1, 2>(out, Cs, Dj, wm, lane);
+  else trsm_product<0, 3>(out, Cs, Dj, wm, lane);
   __syncthreads();
 }
 
@@ -1630,14 +1544,14 @@ __device__ __forceinline__ void tile_trsm(const v4d (&acc)[2][2], const double* 
 // through, every wave's stores complete at the closing barrier
 __device__ __forceinline__ void tile_store(const v4d (&out)[2][2], double* dst, int ld, double* smem) {
   const int tid = opaque_tid(), lane = tid & 63, wave = tid >> 6;
-  const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
+  const int wm = (wave & 1) * 32;
   double(*Cs)[66] = reinterpret_cast<double(*)[66]>(smem);
 #pragma unroll
   for (int bm = 0; bm < 2; ++bm)
 #pragma unroll
     for (int bn = 0; bn < 2; ++bn)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) Cs[wn + 16 * bn + (lane & 15)][wm + 16 * bm + (lane >> 4) + 4 * v] = out[bm][bn][v];
+      for (int v = 0; v < 4; ++v) Cs[tile_col<true>(wave, bn) + (lane & 15)][wm + 16 * bm + (lane >> 4) + 4 * v] = out[bm][bn][v];
   __syncthreads();
   for (int idx = tid; idx < 4096; idx += 256) {
     const int r = idx & 63, c = idx >> 6;
@@ -1647,176 +1561,217 @@ __device__ __forceinline__ void tile_store(const v4d (&out)[2][2], double* dst, 
   __syncthreads();
 }
 
-// dst = X (a 64x64 tile, leading dimension ld) and acc -= X X^T, for X held
-// in accumulator layout (column blocks cb0, cb1 of this wave's rows).  X goes to LDS transposed, T[kk][m] = X(m, kk), so
-// that each of its columns is contiguous there: the stores (written through)
-// leave from LDS as whole columns, and the products read the same copy.
-// Every wave's stores are complete at the closing barrier.
-__device__ __forceinline__ void tile_store_syrk(v4d (&acc)[2][2], const v4d (&X)[2][2], int cb0, int cb1,
-                                                double* __restrict__ dst, size_t ld, double* smem) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
-  double(*T)[66] = reinterpret_cast<double(*)[66]>(smem);
+// The walker's tile (j+1,j+1) by 16x16 blocks on and below the diagonal, three
+// on waves 0 and 3 and two on waves 1 and 2, in MFMA layout: waves 0 and 3 have
+// (B+1,B), (B+1,B+1), (B,B) with B = 0, 2; waves 1 and 2 (R,0), (R,1) with R = 2, 3.
+struct DiagBlocks {
+  v4d b[3];
+};
+__device__ __forceinline__ bool diag_three(int wave) { return wave == 0 || wave == 3; }
+__device__ __forceinline__ int diag_block_row(int wave, int n) { return diag_three(wave) ? (wave & 2) + (n < 2) : 1 + wave; }
+__device__ __forceinline__ int diag_block_col(int wave, int n) { return diag_three(wave) ? (wave & 2) + (n == 1) : n; }
+__device__ __forceinline__ int diag_block_count(int wave) { return diag_three(wave) ? 3 : 2; }
+__device__ __forceinline__ void diag_blocks_load(DiagBlocks& t, const double* src) {
+  const int tid = opaque_tid(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 #pragma unroll
-  for (int bm = 0; bm < 2; ++bm)
+  for (int n = 0; n < 3; ++n)
+    if (n < diag_block_count(wave)) {
+      const double* e = src + part_at(diag_block_row(wave, n), diag_block_col(wave, n), 0) + lane;
 #pragma unroll
-    for (int bn = 0; bn < 2; ++bn)
-#pragma unroll
-      for (int v = 0; v < 4; ++v)
-        T[16 * (bn ? cb1 : cb0) + (lane & 15)][wm + 16 * bm + (lane >> 4) + 4 * v] = X[bm][bn][v];
-  __syncthreads();
-  // 64 columns of 32 row pairs: 32 consecutive threads store one column
-#pragma unroll
-  for (int p = tid; p < 2048; p += 256) {
-    const int c = p >> 5, r = 2 * (p & 31);
-    const double2 x = *reinterpret_cast<const double2*>(&T[c][r]);
-    wt_store(dst + (size_t)r + (size_t)c * ld, x.x);
-    wt_store(dst + (size_t)r + 1 + (size_t)c * ld, x.y);
-  }
-  double a0[16], a1[16], b0[16], b1[16];  // every step's operands read ahead of the MFMAs
-#pragma unroll
-  for (int st = 0; st < 16; ++st) {
-    const int kr = 4 * st + (lane >> 4);
-    a0[st] = T[kr][wm + (lane & 15)];
-    a1[st] = T[kr][wm + 16 + (lane & 15)];
-    b0[st] = T[kr][wn + (lane & 15)];
-    b1[st] = T[kr][wn + 16 + (lane & 15)];
-  }
-  tile_negate(acc);  // adds the products to the negated tile (exact)
-#pragma unroll
-  for (int st = 0; st < 16; ++st) {
-    acc[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0[st], b0[st], acc[0][0], 0, 0, 0);
-    acc[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0[st], b1[st], acc[0][1], 0, 0, 0);
-    acc[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1[st], b0[st], acc[1][0], 0, 0, 0);
-    acc[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1[st], b1[st], acc[1][1], 0, 0, 0);
-  }
-  tile_negate(acc);
-  wt_stores_done();
-  __syncthreads();
-}
-
-// The walker's L_{j+1,j} = P X^T for output column blocks C0 and C1 of this
-// wave's 32 rows (A operands a0, a1 of P in registers, X = inv(L_jj) in
-// sm.Xs): column block c takes k-steps 0..4c+3 only, X^T being zero below
-// its block diagonal (and zero inside the diagonal blocks below the diagonal).
-template <int C0, int C1>
-__device__ __forceinline__ void walker_lt_product(v4d (&Lt)[2][2], const double (&a0)[16], const double (&a1)[16],
-                                                  const DiagSmem& sm, int lane) {
-  constexpr int S0 = 4 * (C0 + 1), S1 = 4 * (C1 + 1);
-#pragma unroll
-  for (int bm = 0; bm < 2; ++bm)
-#pragma unroll
-    for (int bn = 0; bn < 2; ++bn) Lt[bm][bn] = (v4d){0.0, 0.0, 0.0, 0.0};
-  double b0[S0], b1[S1];  // every step's operands read ahead of the MFMAs
-  const int n0c = 16 * C0 + (lane & 15), n1c = 16 * C1 + (lane & 15);
-#pragma unroll
-  for (int st = 0; st < S1; ++st) {
-    const int kr = 4 * st + (lane >> 4);
-    if (st < S0) b0[st < S0 ? st : 0] = sm.Xs[n0c][kr];
-    b1[st] = sm.Xs[n1c][kr];
-  }
-#pragma unroll
-  for (int st = 0; st < S1; ++st) {
-    if (st < S0) {
-      Lt[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0[st], b0[st < S0 ? st : 0], Lt[0][0], 0, 0, 0);
-      Lt[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1[st], b0[st < S0 ? st : 0], Lt[1][0], 0, 0, 0);
+      for (int v = 0; v < 4; ++v) t.b[n][v] = wt_load(e + 64 * v);
     }
-    Lt[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0[st], b1[st], Lt[0][1], 0, 0, 0);
-    Lt[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1[st], b1[st], Lt[1][1], 0, 0, 0);
+}
+
+// t -= X X^T for X = L_{j+1,j} (transposed in T).  store(0) .. store(15) run
+// between the first half's products (a store is issued while the matrix core is
+// busy; one behind the other the sixteen take as long as the products), then
+// halfway().
+template <class Store, class Halfway>
+__device__ __forceinline__ void column_syrk(DiagBlocks& t, const DiagSmem& sm, Store&& store, Halfway&& halfway) {
+  const int tid = opaque_tid(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+#pragma unroll
+  for (int n = 0; n < 3; ++n) t.b[n] = -t.b[n];  // adds the products to the negated blocks (exact)
+  const bool three = diag_three(wave);
+  const double* k0 = &sm.T[lane >> 4][lane & 15];
+  const int oq = 16 * diag_block_row(wave, 0), op = 16 * diag_block_col(wave, 0), oy1 = 16 * diag_block_col(wave, 1);
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    double x[8], y[8], y1[8];
+#pragma unroll
+    for (int st = 0; st < 8; ++st) {
+      const double* k = k0 + 4 * 66 * (8 * h + st);
+      x[st] = k[oq], y[st] = k[op], y1[st] = k[oy1];
+    }
+#pragma unroll
+    for (int st = 0; st < 8; ++st) {
+      t.b[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[st], y[st], t.b[0], 0, 0, 0);
+      t.b[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[st], y1[st], t.b[1], 0, 0, 0);
+      if (three) t.b[2] = __builtin_amdgcn_mfma_f64_16x16x4f64(y[st], y[st], t.b[2], 0, 0, 0);
+      if (h == 0) {
+        __builtin_amdgcn_sched_barrier(0);
+        store(2 * st);
+        store(2 * st + 1);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    if (h == 0) {
+      halfway();
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+#pragma unroll
+  for (int n = 0; n < 3; ++n) t.b[n] = -t.b[n];
+}
+
+// The walker's L_{j+1,j} = P L_jj^-T for this wave's rows 16w.., transposed and in
+// registers (S: P^T, then L^T): column block c's L_c^T = X_cc S_c^T, then S_c' -=
+// L_c L_c'c^T for c' > c, with the operands read ahead and the independent
+// products interleaved.
+__device__ __forceinline__ void rows_solve(v4d (&S)[4], const DiagSmem& sm, int lane) {
+  const int r = lane & 15, kq = lane >> 4;
+  double xa[4][4], la[4][4][4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) {
+      xa[c][kb] = sm.Xs[16 * c + r][16 * c + 4 * kb + kq];
+#pragma unroll
+      for (int e = c + 1; e < 4; ++e) la[c][e][kb] = sm.P[c][16 * e + r][4 * kb + kq];
+    }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    v4d x = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) x = __builtin_amdgcn_mfma_f64_16x16x4f64(xa[c][kb], S[c][kb], x, 0, 0, 0);
+    S[c] = x;
+    const v4d n = -x;
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+      for (int e = c + 1; e < 4; ++e) S[e] = __builtin_amdgcn_mfma_f64_16x16x4f64(la[c][e][kb], n[kb], S[e], 0, 0, 0);
   }
 }
 
-// The walker (ticket 0; see above)
+// The walker (ticket 0; see above).  A column's chain: the tile into rows, four
+// panels, L_{j+1,j} and X_33's products, L_{j+1,j} L_{j+1,j}^T.  What is not on it
+// is done by the waves that a panel leaves idle.  N = 200: a column takes 14.6 us,
+// 8.3 for the panels, 3.2 for L_{j+1,j}, 3.1 for the last update and the stores
+// (20.4 before: 14 for the panels and the whole inverse, and then its stores, the
+// product with it and the update one after the other).  About as long, 10 us from
+// the inverse's publication, takes the next column's partial tile, two hand-offs
+// away; doing its last term where the tile before it is solved, one hand-off
+// away, needs that workgroup to wait for L_{j+1,j} too and came later (16 us).
+// Little is kept in registers over the panels: with the partial tiles loaded and
+// L_{j+1,j} begun during them, the copies between the two register files cost
+// more (16.9 us) than what they hid.
 __device__ __forceinline__ void dag_walker(const DagArgs& g, double* __restrict__ smem) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
   const int nt = g.nt, ld = g.ld;
   double* __restrict__ A = g.A;
   int* err = g.sync + 1;
   int* flags = g.sync + 2;
   int* pflags = g.sync + 2 + nt * nt;
   int* rec = g.rec;  // the first timed-out wait
-  v4d acc[2][2];
-  // acc: partial sum of the current diagonal tile, already including the
+  // the partial sum of the current diagonal tile, already including the
   // last update (the previous column's L_{j,j-1} L_{j,j-1}^T)
+  DiagBlocks acc = {};
   DiagSmem& sm = *reinterpret_cast<DiagSmem*>(smem);
-  if (tid == 0) wait_flag(&pflags[0], g.gen, err, rec, 0, nt * nt);
+  if (threadIdx.x == 0) {
+    sm.ready = 0;
+    sm.stored = 0;
+    wait_flag(&pflags[0], g.gen, err, rec, 0, nt * nt);
+  }
   __syncthreads();
   wt_seen();
-  tile_load<true>(acc, g.part, 64);
+  diag_blocks_load(acc, g.part);
   for (int j = 0; j < nt; ++j) {
+    const int tid = opaque_tid(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 #pragma unroll
-    for (int bm = 0; bm < 2; ++bm)
-#pragma unroll
-      for (int bn = 0; bn < 2; ++bn)
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-          sm.Ls[wm + 16 * bm + (lane >> 4) + 4 * v][wn + 16 * bn + (lane & 15)] = acc[bm][bn][v];
+    for (int n = 0; n < 3; ++n)
+      if (n < diag_block_count(wave)) {
+        const int r0 = 16 * diag_block_row(wave, n), c0 = 16 * diag_block_col(wave, n);
+        blk_store<65>(&sm.R[r0][c0], acc.b[n], 1.0, lane);
+      }
+    wt_stores_done();  // the previous column's
     __syncthreads();
-    double a[16];
+    double a[16], dg[16];
 #pragma unroll
-    for (int q = 0; q < 16; ++q) a[q] = sm.Ls[lane][16 * wave + q];
-    __syncthreads();
-    // column j+1's partial tiles, (j+1,j) into sa0/sa1 (the A operands of
-    // L_{j+1,j}'s product) and (j+1,j+1) into acc: each wave issues its
-    // share of the loads at the first point where both are published (the
-    // column's start, or a point of slack in the factorization), so that
-    // they land during it; a wave that has not issued them by the end of
-    // the factorization waits for the tiles there.  The loads go to
-    // registers: loads into LDS would hold up every barrier until they land.
-    double sa0[16], sa1[16];
+    for (int q = 0; q < 16; ++q) {
+      a[q] = sm.R[lane][16 * wave + q];
+      dg[q] = sm.R[16 * wave + (lane & 15)][16 * wave + q];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // the previous column's L_{j,j-1}: every wave's stores are behind the barrier
+    if (j > 0 && tid == 192) wt_publish(&flags[j + nt * (j - 1)], g.gen);
     const double* sub_src = g.part + (size_t)(2 * j + 1) * 4096;
     const double* acc_src = g.part + (size_t)(2 * (j + 1)) * 4096;
-    bool issued = j + 1 >= nt;
-    auto issue = [&](bool wait) {
-      if (issued) return;
-      if (wait) {
-        if (lane == 0) {
+    double* dinv = g.dinv + (size_t)j * 4096;
+    double* Ljj = A + 64 * j + (size_t)(64 * j) * ld;
+    const bool more = j + 1 < nt;
+    auto idle = [&](int b) {
+      const int lane = opaque_tid() & 63;
+      // column j+1's partial tiles: a wave without a panel asks whether both are
+      // published, near the end, and tells the others through LDS
+      if (more && wave == (b == 3 ? 0 : 3) && b >= 2 && __builtin_amdgcn_readfirstlane(sm.ready) != j + 1) {
+        const int there =
+            __hip_atomic_load(&pflags[2 * j + 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == g.gen &&
+            __hip_atomic_load(&pflags[2 * (j + 1)], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == g.gen;
+        if (there && lane == 0) sm.ready = j + 1;
+      }
+      // what the column has finished leaves while there is time: the factor's
+      // columns by the panel's wave, the inverse's rows
+      if (b == wave + 1) diag_store_factor(a, dg, Ljj, ld);
+      if (b == 3)
+        for (int n = wave; n < 32; n += 3) diag_store_inverse(sm, dinv, n >> 4, n & 15, lane);
+    };
+    v4d S[4];
+    auto last = [&] {
+      const int lane = opaque_tid() & 63;
+      if (more) {
+        if (lane == 0 && sm.ready != j + 1) {
           wait_flag(&pflags[2 * j + 1], g.gen, err, rec, 0, nt * nt + 2 * j + 1);
           wait_flag(&pflags[2 * (j + 1)], g.gen, err, rec, 0, nt * nt + 2 * (j + 1));
         }
-      } else {
-        const int ready =
-            __hip_atomic_load(&pflags[2 * j + 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == g.gen &&
-            __hip_atomic_load(&pflags[2 * (j + 1)], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == g.gen;
-        if (!__builtin_amdgcn_readfirstlane(ready)) return;
+        wt_seen();
+        // (j+1,j) into S, this wave's rows, transposed; (j+1,j+1) into acc
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) S[c][v] = wt_load(sub_src + part_at(c, wave, v) + lane);
+        diag_blocks_load(acc, acc_src);
       }
-      wt_seen();
-      tile_load_a(sa0, sa1, sub_src);
-      tile_load<true>(acc, acc_src, 64);
-      issued = true;
+#pragma unroll
+      for (int n = 0; n < 4; ++n) diag_store_inverse(sm, dinv, 2, 4 * wave + n, lane);
     };
-    issue(false);
-    // the previous column's L_{j,j-1}: published by the last wave, which
-    // waits for the first panel's pivots anyway (its stores are behind the
-    // barriers above)
-    if (j > 0 && tid == 192) wt_publish(&flags[j + nt * (j - 1)], g.gen);
-    diag_factor64(a, sm, 64 * j, [&](int) { issue(false); });
-    diag_store_inverse(sm, g.dinv + (size_t)j * 4096, g.info);
-    wt_stores_done();
+    diag_factor64(a, dg, sm, 64 * j, idle, last);
+    if (more) {
+      const int lane = opaque_tid() & 63;
+      rows_solve(S, sm, lane);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) blk_store<66>(&sm.T[16 * c][16 * wave], S[c], 1.0, lane);
+    }
     __syncthreads();
-    if (tid == 0) wt_publish(&flags[j + nt * j], g.gen);
-    diag_store_factor(sm, A, ld, 64 * j);  // read by nobody in this launch
-    if (j + 1 == nt) break;
-    issue(true);
-    __builtin_amdgcn_s_waitcnt(kWaitVm0);
-    __syncthreads();
-    // L_{j+1,j} = P_{j+1,j} X^T with X = inv(L_jj) still in sm.Xs (lower
-    // blocks).  X^T is block upper triangular, so output column block c
-    // takes only the k-steps of blocks 0..c; waves 0,1 form column blocks
-    // 0 and 3, waves 2,3 blocks 1 and 2: 40 MFMAs each instead of 64
-    v4d Lt[2][2];
-    if (wave >> 1)
-      walker_lt_product<1, 2>(Lt, sa0, sa1, sm, lane);
-    else
-      walker_lt_product<0, 3>(Lt, sa0, sa1, sm, lane);
-    __syncthreads();
-    // L_{j+1,j} out (written through), and the last update of the next
-    // diagonal tile, the stores' completion waited for at the end
-    const int cb0 = (wave >> 1) ? 1 : 0, cb1 = (wave >> 1) ? 2 : 3;
-    tile_store_syrk(acc, Lt, cb0, cb1, A + 64 * (j + 1) + (size_t)(64 * j) * ld, ld, smem);
-    // L_{j+1,j} is published at the start of the next column by a wave
-    // that is idle there
+    if (tid == 0 && sm.bad != 0x7fffffff) atomicMin(g.info, sm.bad);
+#pragma unroll
+    for (int n = 0; n < 4; ++n) diag_store_inverse(sm, dinv, 3, 4 * wave + n, lane);
+    // the inverse is published by the last wave whose stores are complete
+    auto stored = [&] {
+      if (lane == 0 && atomicAdd(&sm.stored, 1) == 4 * j + 3) wt_publish(&flags[j + nt * j], g.gen);
+    };
+    if (!more) {
+      if (wave == 3) diag_store_factor(a, dg, Ljj, ld);
+      wt_stores_done();
+      stored();
+      break;
+    }
+    // L_{j+1,j} out (complete at the next column's start)
+    double* e0 = Ljj + 64 + 16 * wave + (lane & 15) + (size_t)(lane >> 4) * ld;
+    column_syrk(acc, sm, [&](int q) { wt_store(e0 + (size_t)(16 * (q >> 2) + 4 * (q & 3)) * ld, S[q >> 2][q & 3]); }, [&] {
+      __builtin_amdgcn_s_waitcnt(wait_vm(16));  // all but L_{j+1,j}'s: stores complete in order
+      stored();
+      if (wave == 3) diag_store_factor(a, dg, Ljj, ld);
+    });
+    // L_{j+1,j} is published at the start of the next column
   }
 }
 
@@ -1854,8 +1809,8 @@ __device__ __forceinline__ void dag_task(const DagArgs& g, int t, double* __rest
       __syncthreads();
       wt_seen();
       tile_load<true>(acc, g.dinv + (size_t)J * 4096, 64);
-      tile_store_direct(acc, X + 64 * jj + (size_t)(64 * jj) * ldx, ldx);
-      tile_store_direct_t(acc, xdT + (size_t)jj * 4096, 64);
+      tile_store_direct<false>(acc, X + 64 * jj + (size_t)(64 * jj) * ldx, ldx);
+      tile_store_direct_t<false>(acc, xdT + (size_t)jj * 4096, 64);
       wt_stores_done();
       __syncthreads();
       if (tid == 0) wt_publish(&flags[xf + jj + ns * jj], g.gen);
@@ -1931,13 +1886,18 @@ __device__ __forceinline__ void dag_task(const DagArgs& g, int t, double* __rest
         r -= o;
       }
     }
-    tile_load(acc, A + 64 * i + (size_t)(64 * j) * ld, ld);
+    // (the walker takes the tile (j+1,j) transposed)
+    const bool tr = i == j + 1;
+    const double* src = A + 64 * i + (size_t)(64 * j) * ld;
+    if (tr) tile_load_t(acc, src, ld);
+    else tile_load(acc, src, ld);
     // partial sums for the walker: (j,j) without its last term, (j+1,j) complete
-    T = Terms{0, i == j ? max(j - 1, 0) : j, A + 64 * i, A + 64 * i, A + 64 * j, ld, ld, ld, i, nt, j, nt};
+    const int r1 = tr ? j : i, r2 = tr ? i : j;
+    T = Terms{0, i == j ? max(j - 1, 0) : j, A + 64 * r1, A + 64 * r1, A + 64 * r2, ld, ld, ld, r1, nt, r2, nt};
   }
   pair_accumulate(acc, T, flags, g.gen, err, smem, rec, t);
   if (!is_x && i - j <= 1) {
-    tile_store_direct(acc, g.part + (size_t)(2 * j + (i - j)) * 4096, 64);
+    part_store(acc, g.part + (size_t)(2 * j + (i - j)) * 4096);
     wt_stores_done();
     __syncthreads();
     if (tid == 0) wt_publish(&pflags[2 * j + (i - j)], g.gen);
@@ -1953,8 +1913,8 @@ __device__ __forceinline__ void dag_task(const DagArgs& g, int t, double* __rest
   if (is_x) {
     // X_ij^T into the upper block (j,i) for the later tiles of block column j;
     // X_ij into the lower block (i,j)
-    tile_store_direct(out, X + 64 * j + (size_t)(64 * i) * ldx, ldx);
-    tile_store_direct_t(out, X + 64 * i + (size_t)(64 * j) * ldx, ldx);
+    tile_store_direct<true>(out, X + 64 * j + (size_t)(64 * i) * ldx, ldx);
+    tile_store_direct_t<true>(out, X + 64 * i + (size_t)(64 * j) * ldx, ldx);
     wt_stores_done();
     __syncthreads();
     if (tid == 0) wt_publish(&flags[xf + i + ns * j], g.gen);
@@ -2022,10 +1982,10 @@ constexpr int kMacroTiles = 136;
 // The persistent workgroups of a launch of nt block columns: at most one per CU,
 // and no more than its tile work keeps busy beside the diagonal chain, so that
 // concurrent suspensions' factorisations share the chip (a workgroup takes all
-// of a CU's registers).  Fewest workgroups at which a launch alone is no
-// slower: 32 at 19 block columns, 64 at 32 and 35, 96 at 48, 160 at 58 and 60;
-// more than 160 at 88.  A batch of 12 suspensions of N = 108..640 takes 59.6 ms
-// so, and 64.2 with every launch on all CUs.
+// of a CU's registers).  Launches alone, us with 16 + nt^2/24 / 20 + nt^2/16 / 64 +
+// nt^2/6: 19 block columns (N = 108) 420 / 360 / 362, 35 (N = 200) 681 / 600 / 606,
+// 58 (N = 333) 1118 / 1009 / 1015, 88 (N = 512) 2105 / 2075 / 2079 with the
+// inverse; a batch of 12 suspensions of N = 108..640 takes 53.5 / 54.4 / 56.0 ms.
 static int dag_cus() {
   static int n = 0;
   if (n == 0) {
@@ -2039,7 +1999,7 @@ static int dag_cus() {
   return n;
 }
 
-static int dag_workgroups(int nt) { return std::min(dag_cus(), 16 + nt * nt / 24); }
+static int dag_workgroups(int nt) { return std::min(dag_cus(), 20 + nt * nt / 16); }
 
 __global__ void dag_wait_reset_kernel(int* err, int* rec) {
   if (threadIdx.x == 0) *err = 0;

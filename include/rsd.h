@@ -296,7 +296,7 @@ int rsd_ctx_set_resistance_route(rsd_ctx* ctx, int route);
 int rsd_ctx_set_iterative(rsd_ctx* ctx, int precond, double tol, int max_iter, int inner_iters);
 /* on = 1 (the default): the mixed preconditioners' FP32 inner GMRES is captured
  * once as a HIP graph and replayed (one host launch per inner solve in place
- * of about 13 per inner iteration); 0: launched kernel by kernel.  The two
+ * of five per inner iteration); 0: launched kernel by kernel.  The two
  * perform the same arithmetic. */
 int rsd_ctx_set_iterative_graphs(rsd_ctx* ctx, int on);
 /* The last step's total GMRES iterations, its largest final relative residual,

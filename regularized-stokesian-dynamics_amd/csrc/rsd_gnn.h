@@ -79,7 +79,7 @@ struct GnnWork {
   float* gpart = nullptr;  // split reductions
   double* zv = nullptr;    // nz Gaussian vectors (11N each)
   double* gv = nullptr;    // nz vectors K^T (K P z - z)
-  double* wv = nullptr;    // work: 5 vectors
+  double* wv = nullptr;    // work: 4 nz vectors
   double* red = nullptr;   // reductions (2)
   double* hred = nullptr;  // pinned copy
 };

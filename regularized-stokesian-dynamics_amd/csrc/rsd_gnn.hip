@@ -380,30 +380,44 @@ __global__ __launch_bounds__(128) void gnn_out_kernel(LubBsr<double> L, const fl
 }
 
 // ------------------------------------------------------------- the loss
-// out = x with the rows of one field set zeroed: keep_p keeps rows < 6N
-__global__ void keep_rows_kernel(int n, int n6, const double* __restrict__ x, double* __restrict__ y, int keep_p) {
+// All vectors in one launch each, vector blockIdx.y at stride ld: one after the
+// other the loss's products and vector kernels took 330 us for four vectors at
+// N = 256, and 100 so.
+// r -= z; t = r's rows < 6N, zero below
+__global__ void loss_residual_kernel(int n, int n6, size_t ld, const double* __restrict__ z, double* __restrict__ r,
+                                     double* __restrict__ t) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  y[i] = ((i < n6) == (keep_p != 0)) ? x[i] : 0.0;
+  const size_t at = blockIdx.y * ld + i;
+  const double v = r[at] - z[blockIdx.y * (size_t)n + i];
+  r[at] = v;
+  t[at] = i < n6 ? v : 0.0;
 }
-__global__ void axpby_kernel(int n, double a, const double* __restrict__ x, double b, const double* __restrict__ y,
-                             double* __restrict__ out) {
+// y += r's rows >= 6N
+__global__ void add_q_kernel(int n, int n6, size_t ld, const double* __restrict__ r, double* __restrict__ y) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) out[i] = a * x[i] + b * y[i];
+  if (i >= n6 && i < n) y[blockIdx.y * ld + i] += r[blockIdx.y * ld + i];
 }
-// acc[0] += |r|^2, acc[1] += |z|^2 (one workgroup, fixed-order tree)
-__global__ __launch_bounds__(256) void sumsq2_kernel(int n, const double* __restrict__ r, const double* __restrict__ z,
-                                                     double* __restrict__ acc) {
-  __shared__ double s1[256], s2[256];
+// g += t
+__global__ void add_kernel(int n, size_t ld, const double* __restrict__ t, double* __restrict__ g) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) g[blockIdx.y * (size_t)n + i] += t[blockIdx.y * ld + i];
+}
+// acc[0] = sum |r|^2, acc[1] = sum |z|^2 (one workgroup, fixed-order tree)
+__global__ __launch_bounds__(1024) void sumsq2_kernel(int n, int nz, size_t ld, const double* __restrict__ r,
+                                                      const double* __restrict__ z, double* __restrict__ acc) {
+  __shared__ double s1[1024], s2[1024];
   double a = 0.0, b = 0.0;
-  for (int i = threadIdx.x; i < n; i += 256) {
-    a = fma(r[i], r[i], a);
-    b = fma(z[i], z[i], b);
-  }
+  for (int k = 0; k < nz; ++k)
+    for (int i = threadIdx.x; i < n; i += 1024) {
+      const double rv = r[k * ld + i], zv = z[k * (size_t)n + i];
+      a = fma(rv, rv, a);
+      b = fma(zv, zv, b);
+    }
   s1[threadIdx.x] = a;
   s2[threadIdx.x] = b;
   __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
+  for (int w = 512; w > 0; w >>= 1) {
     if (threadIdx.x < w) {
       s1[threadIdx.x] += s1[threadIdx.x + w];
       s2[threadIdx.x] += s2[threadIdx.x + w];
@@ -411,14 +425,8 @@ __global__ __launch_bounds__(256) void sumsq2_kernel(int n, const double* __rest
     __syncthreads();
   }
   if (threadIdx.x == 0) {
-    acc[0] += s1[0];
-    acc[1] += s2[0];
-  }
-}
-__global__ void zero2_kernel(double* acc) {
-  if (threadIdx.x == 0) {
-    acc[0] = 0.0;
-    acc[1] = 0.0;
+    acc[0] = s1[0];
+    acc[1] = s2[0];
   }
 }
 
@@ -749,7 +757,7 @@ int gnn_work_reserve(GnnWork& w, int N, int cap, int nz) {
   RSD_HIP(hipMalloc(&w.gpart, nparts * sizeof(float)));
   RSD_HIP(hipMalloc(&w.zv, (size_t)nz * n * sizeof(double)));
   RSD_HIP(hipMalloc(&w.gv, (size_t)nz * n * sizeof(double)));
-  RSD_HIP(hipMalloc(&w.wv, 5 * n * sizeof(double)));
+  RSD_HIP(hipMalloc(&w.wv, 4 * (size_t)nz * (n + 1) * sizeof(double)));
   RSD_HIP(hipMalloc(&w.red, 2 * sizeof(double)));
   RSD_HIP(hipHostMalloc(&w.hred, 2 * sizeof(double)));
   w.N = N;
@@ -808,35 +816,32 @@ int gnn_loss_grad(GnnWork& w, const float* params, const LubBsr<double>& L, cons
     set_error("gnn_loss_grad: nz outside the reserved buffers");
     return RSD_ERR_ARG;
   }
-  const dim3 blk(256), grd((n + 255) / 256);
+  const dim3 blk(256), grd((n + 255) / 256, nz);
+  // nz vectors of each, an even number of elements apart
+  const size_t nv = ((size_t)n + 1) & ~(size_t)1;
   double* y = w.wv;
-  double* r = w.wv + n;
-  double* kw = w.wv + 2 * (size_t)n;  // apply_k's scratch
-  double* t = w.wv + 4 * (size_t)n;
-  hipLaunchKernelGGL(zero2_kernel, dim3(1), dim3(64), 0, s, w.red);
-  for (int z = 0; z < nz; ++z) {
-    double* Zz = w.zv + (size_t)z * n;
-    RSD_TRY(launch_brown_normal(n, seed, draw * 4096ull + (unsigned long long)z, Zz, s));
-    // r = K P z - z
-    RSD_TRY(block_apply<double>(N, dinv, corr, &L, Zz, y, s));
-    RSD_TRY(apply_k<double>(L, M, ld, y, r, kw, s));
-    hipLaunchKernelGGL(axpby_kernel, grd, blk, 0, s, n, 1.0, (const double*)r, -1.0, (const double*)Zz, r);
-    hipLaunchKernelGGL(sumsq2_kernel, dim3(1), blk, 0, s, n, (const double*)r, (const double*)Zz, w.red);
-    if (!grad) continue;
+  double* mw = y + w.nz * nv;
+  double* r = mw + w.nz * nv;
+  double* t = r + w.nz * nv;
+  for (int z = 0; z < nz; ++z)
+    RSD_TRY(launch_brown_normal(n, seed, draw * 4096ull + (unsigned long long)z, w.zv + (size_t)z * n, s));
+  // r = K P z - z
+  RSD_TRY(block_apply_many(N, dinv, corr, L, w.zv, n, y, nv, nz, s));
+  RSD_TRY(apply_k_many(L, M, ld, y, r, mw, nv, nz, s));
+  hipLaunchKernelGGL(loss_residual_kernel, grd, blk, 0, s, n, n6, nv, (const double*)w.zv, r, t);
+  hipLaunchKernelGGL(sumsq2_kernel, dim3(1), dim3(1024), 0, s, n, nz, nv, (const double*)r, (const double*)w.zv, w.red);
+  if (grad) {
     // G = K^T r = r_P + M (R_lub r_P + r_Q)
-    double* Gz = w.gv + (size_t)z * n;
-    hipLaunchKernelGGL(keep_rows_kernel, grd, blk, 0, s, n, n6, (const double*)r, t, 1);
-    RSD_TRY(bsr_apply<double>(L, t, y, false, s));
-    hipLaunchKernelGGL(keep_rows_kernel, grd, blk, 0, s, n, n6, (const double*)r, kw, 0);
-    hipLaunchKernelGGL(axpby_kernel, grd, blk, 0, s, n, 1.0, (const double*)y, 1.0, (const double*)kw, y);
-    RSD_TRY(dense_gemv<double>(M, ld, n, y, Gz, s));
-    hipLaunchKernelGGL(axpby_kernel, grd, blk, 0, s, n, 1.0, (const double*)Gz, 1.0, (const double*)t, Gz);
+    RSD_TRY(bsr_apply_many(L, t, y, nv, nz, s));
+    hipLaunchKernelGGL(add_q_kernel, grd, blk, 0, s, n, n6, nv, (const double*)r, y);
+    RSD_TRY(dense_gemv_many(M, ld, n, y, nv, w.gv, n, nz, s));
+    hipLaunchKernelGGL(add_kernel, grd, blk, 0, s, n, nv, (const double*)t, w.gv);
   }
   RSD_HIP(hipGetLastError());
   if (grad) {
     const size_t NH = (size_t)N * kGnnH;
     const int chunk = grad_chunk(N), parts = (N + chunk - 1) / chunk;
-    hipLaunchKernelGGL(gnn_dout_kernel, dim3(N), blk, 0, s, L, (const double*)w.pa, (const double*)w.pb,
+    hipLaunchKernelGGL(gnn_dout_kernel, dim3(N), dim3(256), 0, s, L, (const double*)w.pa, (const double*)w.pb,
                        (const double*)w.gv, (const double*)w.zv, nz, (const double*)w.red, log_loss ? 1 : 0,
                        (const float*)w.OUT, w.dOUT);
     GnnBwd b{w.H, w.U, w.V, w.feat, w.dOUT, w.rev};

@@ -83,6 +83,16 @@ template <typename T>
 int block_apply(int N, const T* dinv, const double* corr, const LubBsr<double>* Lcorr, const T* v, T* z,
                 hipStream_t s);
 
+// The same for nz FP64 vectors, with one read of M for up to four of them
+// (strides in elements; even ones and 16-byte aligned vectors are fastest).
+int dense_gemv_many(const double* M, int ld, int n, const double* x, size_t ldx, double* y, size_t ldy, int nz,
+                    hipStream_t s);
+int apply_k_many(const LubBsr<double>& L, const double* M, int ld, const double* x, double* y, double* wbuf, size_t ldv,
+                 int nz, hipStream_t s);
+int bsr_apply_many(const LubBsr<double>& L, const double* w, double* lw, size_t ldv, int nz, hipStream_t s);
+int block_apply_many(int N, const double* dinv, const double* corr, const LubBsr<double>& Lcorr, const double* v,
+                     size_t ldv, double* z, size_t ldz, int nz, hipStream_t s);
+
 struct GmresResult {
   int iterations = 0;
   double relres = 0.0;  // final relative residual ||b - K x|| / ||b|| (recomputed)

@@ -107,6 +107,74 @@ __global__ __launch_bounds__(256) void sym_gemv_kernel(const T* __restrict__ M, 
   if (c < C && c0 + c < n) y[c0 + c] = (red[0][c] + red[1][c]) + (red[2][c] + red[3][c]);
 }
 
+// The same for NZ vectors (strides ldx, ldy) with one read of M, each vector's
+// sums in the same order.  N = 256, four vectors: 52 us one by one, 20 so.
+template <int NZ>
+__global__ __launch_bounds__(256) void sym_gemv_many_kernel(const double* __restrict__ M, size_t ld, int n,
+                                                            const double* __restrict__ x, size_t ldx,
+                                                            double* __restrict__ y, size_t ldy) {
+  constexpr int C = kGemvCols;
+  __shared__ double red[4][C * NZ];
+  const int c0 = blockIdx.x * C, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const double* col[C];
+#pragma unroll
+  for (int c = 0; c < C; ++c) col[c] = M + (size_t)min(c0 + c, n - 1) * ld;
+  double acc[C][NZ];
+#pragma unroll
+  for (int c = 0; c < C; ++c)
+#pragma unroll
+    for (int z = 0; z < NZ; ++z) acc[c][z] = 0.0;
+  const int nv = n / 2 * 2;
+  for (int r = threadIdx.x * 2; r < nv; r += 512) {
+    double2 m[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) m[c] = *reinterpret_cast<const double2*>(col[c] + r);
+#pragma unroll
+    for (int z = 0; z < NZ; ++z) {
+      const double2 xv = *reinterpret_cast<const double2*>(x + z * ldx + r);
+#pragma unroll
+      for (int c = 0; c < C; ++c) acc[c][z] = vec_dot(m[c], xv, acc[c][z]);
+    }
+  }
+  if (nv + (int)threadIdx.x < n) {
+    const int r = nv + threadIdx.x;
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+#pragma unroll
+      for (int z = 0; z < NZ; ++z) acc[c][z] = fma(col[c][r], x[z * ldx + r], acc[c][z]);
+  }
+#pragma unroll
+  for (int c = 0; c < C; ++c)
+#pragma unroll
+    for (int z = 0; z < NZ; ++z) {
+      const double v = wave_sum(acc[c][z]);
+      if (lane == 0) red[wave][c + C * z] = v;
+    }
+  __syncthreads();
+  const int t = threadIdx.x, c = t % C, z = t / C;
+  if (z < NZ && c0 + c < n) y[z * ldy + c0 + c] = (red[0][t] + red[1][t]) + (red[2][t] + red[3][t]);
+}
+
+int dense_gemv_many(const double* M, int ld, int n, const double* x, size_t ldx, double* y, size_t ldy, int nz,
+                    hipStream_t s) {
+  if (ld % 2 || ldx % 2 || ((reinterpret_cast<uintptr_t>(M) | reinterpret_cast<uintptr_t>(x)) & 15)) {
+    for (int z = 0; z < nz; ++z) RSD_TRY(dense_gemv<double>(M, ld, n, x + z * ldx, y + z * ldy, s));
+    return RSD_OK;
+  }
+  const double nn = (double)n * n;
+  for (int z = 0; z < nz; z += 4) {
+    const int k = std::min(4, nz - z);
+    auto kern = k == 4 ? sym_gemv_many_kernel<4>
+                       : k == 3 ? sym_gemv_many_kernel<3> : k == 2 ? sym_gemv_many_kernel<2> : sym_gemv_many_kernel<1>;
+    hipEvent_t pe = prof_begin(kProfGemvSplit64, 2.0 * nn * k, 8.0 * (nn + 2.0 * n * k), s);
+    hipLaunchKernelGGL(kern, dim3((n + kGemvCols - 1) / kGemvCols), dim3(256), 0, s, M, (size_t)ld, n, x + z * ldx, ldx,
+                       y + z * ldy, ldy);
+    prof_end(pe, s);
+  }
+  RSD_HIP(hipGetLastError());
+  return RSD_OK;
+}
+
 template <typename T>
 int dense_gemv(const T* M, int ld, int n, const T* x, T* y, hipStream_t s) {
   constexpr int V = Vec16<T>::n;
@@ -171,7 +239,9 @@ __device__ __forceinline__ void bsr_rows(const LubBsr<T>& L, int g, int lane, co
 // neighbours' dofs (rows < 6 only when nrows is 6)
 template <typename T>
 __global__ __launch_bounds__(64 * kGroup) void bsr_apply_kernel(LubBsr<T> L, const T* __restrict__ w,
-                                                                T* __restrict__ lw, int nrows) {
+                                                                T* __restrict__ lw, int nrows, size_t ldv) {
+  w += blockIdx.y * ldv;  // vector blockIdx.y
+  lw += blockIdx.y * ldv;
   const int g = blockIdx.x * kGroup + (threadIdx.x >> 6), lane = threadIdx.x & 63, N = L.N;
   if (g >= N) return;
   T acc[11];
@@ -184,20 +254,33 @@ __global__ __launch_bounds__(64 * kGroup) void bsr_apply_kernel(LubBsr<T> L, con
 template <typename T>
 int bsr_apply(const LubBsr<T>& L, const T* w, T* lw, bool p_rows_only, hipStream_t s) {
   const int nrows = p_rows_only ? 6 : 11;
-  hipLaunchKernelGGL(bsr_apply_kernel<T>, dim3((L.N + kGroup - 1) / kGroup), dim3(64 * kGroup), 0, s, L, w, lw, nrows);
+  hipLaunchKernelGGL(bsr_apply_kernel<T>, dim3((L.N + kGroup - 1) / kGroup), dim3(64 * kGroup), 0, s, L, w, lw, nrows,
+                     (size_t)0);
+  RSD_HIP(hipGetLastError());
+  return RSD_OK;
+}
+int bsr_apply_many(const LubBsr<double>& L, const double* w, double* lw, size_t ldv, int nz, hipStream_t s) {
+  hipLaunchKernelGGL(bsr_apply_kernel<double>, dim3((L.N + kGroup - 1) / kGroup, nz), dim3(64 * kGroup), 0, s, L, w, lw,
+                     11, ldv);
   RSD_HIP(hipGetLastError());
   return RSD_OK;
 }
 
 // K's rows from w = M x: y_P = x_P + (R_lub w)_P, y_Q = w_Q.  With k > 0 also
 // the workgroup's share of V_j . y for the k vectors V_j (stride ldv), to
-// part[j * gridDim.x + blockIdx.x].
+// part[j * gridDim.x + blockIdx.x]; with k = 0 for gridDim.y vectors x, w, y
+// (stride ldv).
 template <typename T>
 __global__ __launch_bounds__(64 * kGroup) void k_rows_kernel(LubBsr<T> L, const T* __restrict__ x,
                                                              const T* __restrict__ w, T* __restrict__ y, int k,
                                                              const T* __restrict__ V, size_t ldv,
                                                              double* __restrict__ part) {
   __shared__ T ys[11 * kGroup];
+  if (k == 0) {  // vector blockIdx.y of several
+    x += blockIdx.y * ldv;
+    w += blockIdx.y * ldv;
+    y += blockIdx.y * ldv;
+  }
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, N = L.N;
   const int g0 = blockIdx.x * kGroup, g = g0 + wave;
   if (g < N) {
@@ -241,6 +324,15 @@ static int apply_k_dots(const LubBsr<T>& L, const T* M, int ld, const T* x, T* y
 template <typename T>
 int apply_k(const LubBsr<T>& L, const T* M, int ld, const T* x, T* y, T* wbuf, hipStream_t s) {
   return apply_k_dots<T>(L, M, ld, x, y, wbuf, 0, nullptr, 0, nullptr, s);
+}
+
+int apply_k_many(const LubBsr<double>& L, const double* M, int ld, const double* x, double* y, double* wbuf, size_t ldv,
+                 int nz, hipStream_t s) {
+  RSD_TRY(dense_gemv_many(M, ld, 11 * L.N, x, ldv, wbuf, ldv, nz, s));
+  hipLaunchKernelGGL(k_rows_kernel<double>, dim3(k_rows_groups(L.N), nz), dim3(64 * kGroup), 0, s, L, x,
+                     (const double*)wbuf, y, 0, (const double*)nullptr, ldv, (double*)nullptr);
+  RSD_HIP(hipGetLastError());
+  return RSD_OK;
 }
 
 // ----------------------------------------------------------- block Jacobi
@@ -341,7 +433,10 @@ __global__ __launch_bounds__(64 * kGroup) void block_apply_kernel(int N, const T
                                                                   const double* __restrict__ corr, LubBsr<double> Lc,
                                                                   const T* __restrict__ v, T* __restrict__ z, int np,
                                                                   const double* __restrict__ partn,
-                                                                  T* __restrict__ norm, double* __restrict__ inv) {
+                                                                  T* __restrict__ norm, double* __restrict__ inv,
+                                                                  size_t ldv, size_t ldz) {
+  v += blockIdx.y * ldv;  // vector blockIdx.y
+  z += blockIdx.y * ldz;
   const int g = blockIdx.x * kGroup + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (g >= N) return;
   const int nn = corr ? Lc.nnb[g] : 0;
@@ -394,7 +489,14 @@ static int block_apply_scaled(int N, const T* dinv, const double* corr, const Lu
   LubBsr<double> Lc{};
   if (corr && Lcorr) Lc = *Lcorr;
   hipLaunchKernelGGL(block_apply_kernel<T>, dim3((N + kGroup - 1) / kGroup), dim3(64 * kGroup), 0, s, N, dinv,
-                     (corr && Lcorr) ? corr : nullptr, Lc, v, z, np, partn, norm, inv);
+                     (corr && Lcorr) ? corr : nullptr, Lc, v, z, np, partn, norm, inv, (size_t)0, (size_t)0);
+  RSD_HIP(hipGetLastError());
+  return RSD_OK;
+}
+int block_apply_many(int N, const double* dinv, const double* corr, const LubBsr<double>& Lcorr, const double* v,
+                     size_t ldv, double* z, size_t ldz, int nz, hipStream_t s) {
+  hipLaunchKernelGGL(block_apply_kernel<double>, dim3((N + kGroup - 1) / kGroup, nz), dim3(64 * kGroup), 0, s, N, dinv,
+                     corr, Lcorr, v, z, 0, (const double*)nullptr, (double*)nullptr, (double*)nullptr, ldv, ldz);
   RSD_HIP(hipGetLastError());
   return RSD_OK;
 }

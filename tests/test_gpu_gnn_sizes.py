@@ -41,6 +41,29 @@ def reference(p, M, R, nnb, col, dist, radii, Z):
     return float(loss.detach()), pt.grad.numpy()
 
 
+@pytest.mark.parametrize("nz", [1, 2, 4, 5, 8])
+def test_numbers_of_vectors(rsd, nz):
+    """The products for several vectors at once, in groups of up to four, and vectors of odd length (11 * 33)."""
+    from rsd_amd.configs import random_suspension
+    conf, radii, L = random_suspension(33, 0.35, 22)
+    sus = rsd.Suspension(conf, radii, rsd.default_config(L))
+    sus.prepare_iterative(0.0)
+    M, R, nnb, col, dist, cap = sus.iterative_system()
+    gnn = rsd.Gnn(seed=4)
+    p = gnn.params()
+    p[-133:] = (0.05 * np.random.default_rng(6).standard_normal(133)).astype(np.float32)
+    gnn.set_params(p)
+    loss, grad, Z = sus.gnn_loss(gnn, nz=nz, seed=12)
+    want, gwant = reference(p, M, R, nnb, col, dist, radii, Z)
+    only, _, _ = sus.gnn_loss(gnn, nz=nz, seed=12, grad=False)
+    assert only == loss
+    # bounds as below
+    assert abs(loss - want) <= 5.5e-5 * want
+    assert relerr(gwant, grad) < 1e-3
+    gnn.close()
+    sus.close()
+
+
 @pytest.mark.parametrize("n,phi", [(1, 0.01), (5, 0.01), (9, 0.05), (17, 0.4), (72, 0.5), (530, 0.3)])
 def test_loss_and_gradient(rsd, n, phi):
     from rsd_amd.configs import random_suspension

@@ -1582,10 +1582,10 @@ __device__ __forceinline__ void diag_blocks_load(DiagBlocks& t, const double* sr
     }
 }
 
-// t -= X X^T for X = L_{j+1,j} (transposed in T).  store(0) .. store(15) run
-// between the first half's products (a store is issued while the matrix core is
-// busy; one behind the other the sixteen take as long as the products), then
-// halfway().
+// t -= X X^T for X = L_{j+1,j} (transposed in T).  halfway() runs after half of
+// the products, store(0) .. store(15) between the others (a store is issued while
+// the matrix core is busy; one behind the other the sixteen take as long as the
+// products).
 template <class Store, class Halfway>
 __device__ __forceinline__ void column_syrk(DiagBlocks& t, const DiagSmem& sm, Store&& store, Halfway&& halfway) {
   const int tid = opaque_tid(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1607,7 +1607,7 @@ __device__ __forceinline__ void column_syrk(DiagBlocks& t, const DiagSmem& sm, S
       t.b[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[st], y[st], t.b[0], 0, 0, 0);
       t.b[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[st], y1[st], t.b[1], 0, 0, 0);
       if (three) t.b[2] = __builtin_amdgcn_mfma_f64_16x16x4f64(y[st], y[st], t.b[2], 0, 0, 0);
-      if (h == 0) {
+      if (h == 1) {
         __builtin_amdgcn_sched_barrier(0);
         store(2 * st);
         store(2 * st + 1);
@@ -1615,6 +1615,7 @@ __device__ __forceinline__ void column_syrk(DiagBlocks& t, const DiagSmem& sm, S
       }
     }
     if (h == 0) {
+      __builtin_amdgcn_sched_barrier(0);
       halfway();
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -1767,7 +1768,7 @@ __device__ __forceinline__ void dag_walker(const DagArgs& g, double* __restrict_
     // L_{j+1,j} out (complete at the next column's start)
     double* e0 = Ljj + 64 + 16 * wave + (lane & 15) + (size_t)(lane >> 4) * ld;
     column_syrk(acc, sm, [&](int q) { wt_store(e0 + (size_t)(16 * (q >> 2) + 4 * (q & 3)) * ld, S[q >> 2][q & 3]); }, [&] {
-      __builtin_amdgcn_s_waitcnt(wait_vm(16));  // all but L_{j+1,j}'s: stores complete in order
+      wt_stores_done();
       stored();
       if (wave == 3) diag_store_factor(a, dg, Ljj, ld);
     });

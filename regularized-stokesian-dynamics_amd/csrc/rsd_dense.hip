@@ -1,9 +1,9 @@
 // rsd_dense.hip -- FP64 dense linear algebra for the grand-resistance solve.
 //
 // Replaces MATREV (matrices.f90:4-34: DPOTRF('U') + DPOTRI('U') + mirror)
-// with a right-looking blocked Cholesky, a recursive triangular inverse and
-// a triangular X^T X product, all built on one batched 64x64-tile GEMM that
-// runs on the CDNA4 FP64 matrix cores (v_mfma_f64_16x16x4_f64).
+// with a dataflow tile Cholesky in one launch, and a recursive triangular
+// inverse and a triangular X^T X product on one batched 64x64-tile GEMM, all
+// on the CDNA4 FP64 matrix cores (v_mfma_f64_16x16x4_f64).
 //
 // Layout: column-major, order padded to a multiple of 64 with an identity
 // block so no kernel needs edge handling.  The symmetric input is read from
@@ -840,8 +840,10 @@ __device__ __forceinline__ void wait_flag(const int* flag, int gen, int* err, in
 // partial tiles of the column it is on.  Other tiles wait only for lower
 // tickets or for the walker; early tiles wait for other tiles, some of
 // higher tickets, but at any time only the early tiles within kAhead
-// columns of the walker's (about 3 kAhead workgroups) can be waiting, so the
-// other tiles always have workgroups to run on.  Every wait is bounded.
+// columns of the walker's can be waiting, so the other tiles always have
+// workgroups to run on: played through task by task, 16 workgroups beside the
+// walker finish every order up to 136 block columns (fewer do not from 10 on),
+// and a launch has 19 at least, or one per task.  Every wait is bounded.
 constexpr int kDagStage = 2 * 8192;  // two staged terms of two 64x64 tiles
 constexpr int kAhead = 6;             // columns by which the early tiles start ahead
 constexpr int kEarly = 3;             // early tiles per column: (c,c), (c+1,c), (c+2,c)

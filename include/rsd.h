@@ -20,6 +20,11 @@
  * definite leading minor (non-fatal, as MATREV prints and continues,
  * matrices.f90:19-24); < 0 an RSD_ERR_* code, with rsd_last_error() text.
  * Nothing is printed.  One host thread per context; calls are blocking.
+ *
+ * The entry points without a context keep memory for a thread's next call: 8 MiB
+ * of pinned host memory, and device memory for what its largest call took, up to
+ * 512 MiB.  The device memory shrinks after 16 to 31 calls that took less than a
+ * quarter of it, and both go when the thread ends.
  */
 #ifndef RSD_H_
 #define RSD_H_

@@ -258,15 +258,20 @@ struct DBuf {
 // Device memory of the host-array entry points: each thread keeps one block and
 // hands it out from the front while a call runs (a hipMalloc and a hipFree a
 // matrix took longer than the algebra at N = 100).  What a call needs beyond
-// the block comes from hipMalloc and goes back at its end; the block then grows
-// to what the call used, up to kArenaMax, at the start of the thread's next
-// call.  The entry points run on the null stream and end with a wait for it, so
-// a call finds the block free.
+// the block comes from hipMalloc and goes back at its end.  At the start of a
+// thread's next call the block grows to what the last one used, up to
+// kArenaMax; when kArenaWindow calls in a row have used less than a quarter of
+// it, it shrinks to the most that they used, and it goes when the thread ends.
+// The entry points run on the null stream and end with a wait for it, so a call
+// finds the block free.
 constexpr size_t kArenaMax = 512u << 20;
+constexpr int kArenaWindow = 16;
 struct DeviceArena {
   int dev = -1, live = 0;
   char* base = nullptr;
   size_t cap = 0, used = 0, total = 0;  // the block's size, its part in use, all that the last call asked for
+  size_t peak = 0;                      // the most that one of the last `calls` calls asked for
+  int calls = 0;
   std::vector<void*> extra;
   ~DeviceArena() { drop(); }
   void drop() {
@@ -274,13 +279,25 @@ struct DeviceArena {
     base = nullptr;
     cap = 0;
   }
+  // the block's size for the next call
+  size_t next_size() {
+    const size_t want = std::min(total, kArenaMax);
+    peak = std::max(peak, want);
+    size_t size = std::max(cap, want);
+    if (++calls >= kArenaWindow) {
+      if (peak < cap / 4) size = peak;
+      peak = 0;
+      calls = 0;
+    }
+    return size;
+  }
   int get(size_t bytes, void** p) {
     bytes = (std::max<size_t>(bytes, 1) + 255) & ~(size_t)255;
     if (live == 0) {
       int d = 0;
       RSD_HIP(hipGetDevice(&d));
-      const size_t want = std::min(total, kArenaMax);
-      if (d != dev || want > cap) {
+      const size_t want = next_size();
+      if (d != dev || want != cap) {
         drop();
         dev = d;
         if (want > 0) {

@@ -22,9 +22,10 @@
  * Nothing is printed.  One host thread per context; calls are blocking.
  *
  * The entry points without a context keep memory for a thread's next call: 8 MiB
- * of pinned host memory, and device memory for what its largest call took, up to
- * 512 MiB.  The device memory shrinks after 16 to 31 calls that took less than a
- * quarter of it, and both go when the thread ends.
+ * of pinned host memory, a workspace on the device of about one matrix of its
+ * largest order, and device memory for what its largest call took, up to 512 MiB.
+ * The last shrinks after 16 to 31 calls that took less than a quarter of it, and
+ * all of them go when the thread ends.
  */
 #ifndef RSD_H_
 #define RSD_H_

@@ -766,9 +766,20 @@ int rsd_lubmxcalc(int n, int nb, int is_period, const double* pos, const double*
   return rc;
 }
 
+// Their workspace, a thread's own: released when the thread ends or goes on
+// to another device.
 static DenseWork& host_api_dense() {
-  static thread_local DenseWork w;
-  return w;
+  struct Owned {
+    int dev = -1;
+    DenseWork w;
+    ~Owned() { dense_release(w); }
+  };
+  static thread_local Owned o;
+  int d = 0;
+  (void)hipGetDevice(&d);
+  if (d != o.dev) dense_release(o.w);
+  o.dev = d;
+  return o.w;
 }
 
 int rsd_matrev(int n, double* a) {

@@ -1,6 +1,7 @@
 """The device memory that the host-array entry points keep between a thread's calls: given back after a run of calls
-that need much less of it."""
+that need much less of it, and all of it when the thread ends."""
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -32,6 +33,22 @@ def test_memory_is_given_back(rsd):
     t.join()
     # the three matrices but for what the small calls need and the driver's granularity
     assert seen["small"] - seen["large"] >= 180 * MIB, seen
+
+
+def test_a_thread_that_ends_keeps_nothing(rsd):
+    A = np.eye(3000)
+    rsd.matrev(np.eye(10))
+    start = free_bytes()
+    for _ in range(3):
+        t = threading.Thread(target=rsd.matrev, args=(A,))
+        t.start()
+        t.join()
+    # (the last destructors run shortly after join() returns; an order of 3000 takes 86 MiB of workspace)
+    for _ in range(100):
+        if start - free_bytes() <= 16 * MIB:
+            break
+        time.sleep(0.05)
+    assert start - free_bytes() <= 16 * MIB, (start, free_bytes())
 
 
 def test_sizes_around_a_shrink(rsd):

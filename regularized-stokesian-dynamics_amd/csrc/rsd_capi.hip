@@ -1002,6 +1002,7 @@ struct rsd_ctx {
   int last_it_iters = 0, last_it_fallback = 0;
   double last_it_relres = 0.0;
   static constexpr int kBsrCap = 96;  // lubrication neighbours per particle the block-sparse rows hold
+  static_assert(kBsrCap <= kIterMaxNeighbours, "the neighbour products hold every neighbour's index");
   DBuf bsr_blk, bsr_self, xit, bit, wit;
   int* bsr_ix = nullptr;   // [0, N) counts, [N, N + N cap) columns, then the overflow word
   float* bsr32 = nullptr;  // FP32 copies: blocks, self blocks, then M

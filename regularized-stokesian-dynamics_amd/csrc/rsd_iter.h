@@ -15,8 +15,12 @@
 
 namespace rsd {
 
+// The most neighbours a particle's block row may hold: a wave's lanes hand
+// their indices round, two each.
+constexpr int kIterMaxNeighbours = 128;
+
 // The lubrication resistance in 11x11 blocks (LubParams::bsr_*), in the
-// precision T of its blocks.
+// precision T of its blocks; cap <= kIterMaxNeighbours neighbours a particle.
 template <typename T>
 struct LubBsr {
   int N = 0, cap = 0;

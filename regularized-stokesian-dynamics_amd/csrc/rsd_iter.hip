@@ -204,6 +204,7 @@ __device__ __forceinline__ NeighbourCols neighbour_cols(const int* col, int cap,
   const int* c = col + (size_t)g * cap;
   return {lane < cap ? c[lane] : 0, 64 + lane < cap ? c[64 + lane] : 0};
 }
+static_assert(kIterMaxNeighbours == 2 * 64, "two neighbours a lane");
 // neighbour q (every lane of the wave active)
 __device__ __forceinline__ int neighbour(const NeighbourCols& nc, int q) {
   const int a = __shfl(nc.lo, q & 63, 64), b = __shfl(nc.hi, q & 63, 64);

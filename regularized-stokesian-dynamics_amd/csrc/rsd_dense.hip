@@ -15,6 +15,7 @@
 #include <cmath>
 #include <vector>
 
+#include "rsd_dag.h"
 #include "rsd_internal.h"
 #include "rsd_prof.h"
 
@@ -839,14 +840,11 @@ __device__ __forceinline__ void wait_flag(const int* flag, int gen, int* err, in
 // cache-wide fence on either side).  The walker waits only for the two
 // partial tiles of the column it is on.  Other tiles wait only for lower
 // tickets or for the walker; early tiles wait for other tiles, some of
-// higher tickets, but at any time only the early tiles within kAhead
-// columns of the walker's can be waiting, so the other tiles always have
-// workgroups to run on: played through task by task, 16 workgroups beside the
-// walker finish every order up to 136 block columns (fewer do not from 10 on),
-// and a launch has 19 at least, or one per task.  Every wait is bounded.
+// higher tickets, but at any time only the early tiles within kAhead columns of
+// the walker's can be waiting, so the other tiles have workgroups to run on as
+// long as kDagBeside of them are resident beside the walker.  Every wait is
+// bounded.
 constexpr int kDagStage = 2 * 8192;  // two staged terms of two 64x64 tiles
-constexpr int kAhead = 6;             // columns by which the early tiles start ahead
-constexpr int kEarly = 3;             // early tiles per column: (c,c), (c+1,c), (c+2,c)
 constexpr int kDiagDoubles = (sizeof(DiagSmem) + 15) / 16 * 2;  // the walker's share, 16-byte aligned
 constexpr int kDagSmemDoubles = kDiagDoubles > kDagStage ? kDiagDoubles : kDagStage;
 static_assert(kDagStage <= kDagSmemDoubles && 2 * 64 * 66 <= kDagSmemDoubles, "staging fits the shared buffer");
@@ -1467,30 +1465,6 @@ __device__ __forceinline__ void macro_task(const DagArgs& g, int I, int J, int t
   publish(j0 + 1);
 }
 
-// Ticket order with macro tasks, per pair J of block columns: the early tiles
-// of columns 2J + kAhead and 2J + 1 + kAhead; tile (2J+3, 2J) alone; the macro
-// tasks (I, J), I >= J + 2; and, when nt is odd, the last block row's two tiles.
-struct MacroCounts {
-  int e0, e1, single, macros, last;
-};
-__host__ __device__ inline int dag_early(int nt, int c) { return c < nt ? (kEarly < nt - c ? kEarly : nt - c) : 0; }
-__host__ __device__ inline MacroCounts macro_counts(int nt, int J) {
-  const int m = nt / 2 - (J + 2);
-  return {dag_early(nt, 2 * J + kAhead), dag_early(nt, 2 * J + 1 + kAhead), 2 * J + 3 < nt ? 1 : 0, m > 0 ? m : 0,
-          (nt & 1) && nt - 1 >= 2 * J + 4 ? 2 : 0};
-}
-// the factorization's tickets after the walker's
-static int dag_tickets(int nt, bool macro) {
-  if (!macro) return nt * (nt + 1) / 2;
-  int n = 0;
-  for (int c = 0; c < kAhead; ++c) n += dag_early(nt, c);
-  for (int J = 0; J < (nt + 1) / 2; ++J) {
-    const MacroCounts k = macro_counts(nt, J);
-    n += k.e0 + k.e1 + k.single + k.macros + k.last;
-  }
-  return n;
-}
-
 // Column blocks C0 < C1 of out = C Dinv^T for this wave's 32 rows: Dinv^T is zero
 // below its block diagonal, so block c takes the k-steps 0 .. 4c+3 only, 40
 // products a wave instead of 64.
@@ -1823,12 +1797,9 @@ __device__ __forceinline__ void dag_task(const DagArgs& g, int t, double* __rest
     // (I = s0 + i).  The sum is accumulated transposed, acc = -sum X_kj^T L_Ik^T,
     // from X_kj^T (kept in X's upper block (j,k); X_jj^T in xdT), so that the
     // solve with Dinv_I is tile_trsm's product: X_ij^T = acc Dinv_I^T.
-    j = r - ns;
-    i = 1;
-    while (j >= i) {
-      j -= i;
-      ++i;
-    }
+    const DagTile q = dag_x_tile(ns, r);
+    i = q.i;
+    j = q.j;
 #pragma unroll
     for (int bm = 0; bm < 2; ++bm)
 #pragma unroll
@@ -1837,58 +1808,13 @@ __device__ __forceinline__ void dag_task(const DagArgs& g, int t, double* __rest
     T = Terms{j, i, xdT + (size_t)j * 4096, X + 64 * j, A + 64 * I + (size_t)(64 * s0) * ld,
               64, ldx, ld, xf + ns * j, 1, I + nt * s0, nt};
   } else {
-    int r = t - 1, c0 = 0;
-    for (; c0 < kAhead && c0 < nt; ++c0) {
-      if (r < dag_early(nt, c0)) break;
-      r -= dag_early(nt, c0);
+    const DagTile q = dag_tile(nt, MACRO, t);
+    if (MACRO && q.macro) {
+      macro_task(g, q.i, q.j, t, smem);
+      return;
     }
-    if (c0 < kAhead && c0 < nt) {
-      j = c0;
-      i = c0 + r;
-    } else if (MACRO) {
-      i = j = 0;
-      for (int J = 0;; ++J) {
-        const MacroCounts k = macro_counts(nt, J);
-        if (r < k.e0 + k.e1) {
-          j = 2 * J + kAhead + (r < k.e0 ? 0 : 1);
-          i = j + (r < k.e0 ? r : r - k.e0);
-          break;
-        }
-        r -= k.e0 + k.e1;
-        if (r < k.single) {
-          j = 2 * J;
-          i = j + 3;
-          break;
-        }
-        r -= k.single;
-        if (r < k.macros) {
-          macro_task(g, J + 2 + r, J, t, smem);
-          return;
-        }
-        r -= k.macros;
-        if (r < k.last) {
-          j = 2 * J + r;
-          i = nt - 1;
-          break;
-        }
-        r -= k.last;
-      }
-    } else {
-      for (j = 0;; ++j) {
-        const int e = dag_early(nt, j + kAhead), o = nt - j - kEarly > 0 ? nt - j - kEarly : 0;
-        if (r < e) {
-          i = j + kAhead + r;
-          j = j + kAhead;
-          break;
-        }
-        r -= e;
-        if (r < o) {
-          i = j + kEarly + r;
-          break;
-        }
-        r -= o;
-      }
-    }
+    i = q.i;
+    j = q.j;
     // (the walker takes the tile (j+1,j) transposed)
     const bool tr = i == j + 1;
     const double* src = A + 64 * i + (size_t)(64 * j) * ld;
@@ -1927,16 +1853,15 @@ __device__ __forceinline__ void dag_task(const DagArgs& g, int t, double* __rest
   }
 }
 
-// The launch is persistent: as many workgroups as the GPU holds at once
-// (one per CU: the tile staging fills the LDS), each taking tickets in turn
-// until they run out.  A task waits only for tasks of lower tickets, for the
-// walker, or (the early tiles, at most kEarly kAhead of them) for tiles of
-// higher tickets; since every ticket taken is held by a running workgroup,
-// and a workgroup takes the next ticket as soon as it is free, the tasks
-// waited for always run.  (With one workgroup per task, the hardware assigns
-// the workgroups to the XCDs in advance: when the only XCD with workgroups
-// left to start is full of waiting ones, the lowest untaken ticket never
-// starts.)
+// The launch is persistent: dag_workgroups() workgroups, at most one per CU (the
+// tile staging fills the LDS), each taking tickets in turn until they run out.
+// A task waits only for tasks of lower tickets, for the walker, or (the early
+// tiles) for tiles of higher tickets; every ticket taken is held by a running
+// workgroup, and a workgroup takes the next ticket as soon as it is free, so
+// with kDagBeside workgroups beside the walker's the tasks waited for always
+// run.  (With one workgroup per task, the hardware assigns the workgroups to the
+// XCDs in advance: when the only XCD with workgroups left to start is full of
+// waiting ones, the lowest untaken ticket never starts.)
 template <bool MACRO>
 __global__ __launch_bounds__(256) void potrf_dag_kernel(DagArgs g) {
   // one LDS variable: with several, the compiler's record of which pointers
@@ -1974,21 +1899,6 @@ __global__ __launch_bounds__(256) void potrf_dag_kernel(DagArgs g) {
   }
 }
 
-// Block columns from which macro tasks take the place of the single tiles away
-// from the diagonal.  Below, a launch has too few of them to fill the CUs near
-// its end; single / macro ms for the 11N launch and the W_PP product after it:
-// N = 640 (110 block columns) 3.71 / 3.76, N = 720 (124) 5.15 / 5.27, N = 800
-// (138) 6.74 / 6.70, N = 900 (155) 9.57 / 9.33, N = 997 (172) 12.6 / 12.3,
-// N = 1400 (242) 35.9 / 33.0.
-constexpr int kMacroTiles = 136;
-
-// The persistent workgroups of a launch of nt block columns: at most one per CU,
-// and no more than its tile work keeps busy beside the diagonal chain, so that
-// concurrent suspensions' factorisations share the chip (a workgroup takes all
-// of a CU's registers).  Launches alone, us with 16 + nt^2/24 / 20 + nt^2/16 / 64 +
-// nt^2/6: 19 block columns (N = 108) 420 / 360 / 362, 35 (N = 200) 681 / 600 / 606,
-// 58 (N = 333) 1118 / 1009 / 1015, 88 (N = 512) 2105 / 2075 / 2079 with the
-// inverse; a batch of 12 suspensions of N = 108..640 takes 53.5 / 54.4 / 56.0 ms.
 static int dag_cus() {
   static int n = 0;
   if (n == 0) {
@@ -2001,8 +1911,6 @@ static int dag_cus() {
   }
   return n;
 }
-
-static int dag_workgroups(int nt) { return std::min(dag_cus(), 20 + nt * nt / 16); }
 
 __global__ void dag_wait_reset_kernel(int* err, int* rec) {
   if (threadIdx.x == 0) *err = 0;
@@ -2065,7 +1973,7 @@ int potrf_lower_x(DenseWork& w, double* A, int n, int ld, int s0, double* X, int
   const double nd = (double)n, md = 64.0 * ns;
   hipEvent_t pe = prof_begin(kProfPotrfDiag, (nd * nd * nd + md * md * md) / 3.0, 0.0, s);
   hipLaunchKernelGGL((macro ? potrf_dag_kernel<true> : potrf_dag_kernel<false>),
-                     dim3(std::min(1 + nfac + ns * (ns + 1) / 2, dag_workgroups(nt))), dim3(256), 0, s, g);
+                     dim3(dag_workgroups(nt, 1 + nfac + ns * (ns + 1) / 2, dag_cus())), dim3(256), 0, s, g);
   prof_end(pe, s);
   RSD_HIP(hipGetLastError());
   return RSD_OK;

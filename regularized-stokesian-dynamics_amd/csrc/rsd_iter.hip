@@ -509,21 +509,18 @@ int block_apply(int N, const T* dinv, const double* corr, const LubBsr<double>* 
 }
 
 // ------------------------------------------------------------ vector kernels
-// h[j] = V_j . w for j < k (one workgroup per j, fixed-order tree in LDS)
-template <typename T>
-__global__ __launch_bounds__(256) void multi_dot_kernel(const T* __restrict__ V, size_t ldv, int n,
-                                                        const T* __restrict__ w, T* __restrict__ h) {
+// h[0] = v . v (one workgroup, fixed-order tree in LDS)
+__global__ __launch_bounds__(256) void squared_norm_kernel(int n, const double* __restrict__ v, double* __restrict__ h) {
   __shared__ double red[256];
-  const T* v = V + (size_t)blockIdx.x * ldv;
   double a = 0.0;
-  for (int i = threadIdx.x; i < n; i += 256) a = fma((double)v[i], (double)w[i], a);
+  for (int i = threadIdx.x; i < n; i += 256) a = fma(v[i], v[i], a);
   red[threadIdx.x] = a;
   __syncthreads();
   for (int s = 128; s > 0; s >>= 1) {
     if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
     __syncthreads();
   }
-  if (threadIdx.x == 0) h[blockIdx.x] = (T)red[0];
+  if (threadIdx.x == 0) h[0] = red[0];
 }
 
 // The two passes of classical Gram-Schmidt of w against V_0..V_{k-1} (unit
@@ -623,13 +620,12 @@ static int orthogonalise(const T* V, size_t ldv, int n, int k, const OrthoWork& 
   return RSD_OK;
 }
 
-// y = (T) x, and the partial sums of the squared norm of y
-template <typename Tin, typename T>
-__global__ __launch_bounds__(kVecRows) void krylov_start_kernel(int n, const Tin* __restrict__ x, T* __restrict__ y,
-                                                                double* __restrict__ partn) {
+// y = (float) x, and the partial sums of the squared norm of y
+__global__ __launch_bounds__(kVecRows) void krylov_start_kernel(int n, const double* __restrict__ x,
+                                                                float* __restrict__ y, double* __restrict__ partn) {
   __shared__ double red[4];
   const int i = blockIdx.x * kVecRows + threadIdx.x, lane = threadIdx.x & 63;
-  const T v = i < n ? (T)x[i] : (T)0;
+  const float v = i < n ? (float)x[i] : 0.0f;
   if (i < n) y[i] = v;
   const double s = wave_sum((double)v * (double)v);
   if (lane == 0) red[threadIdx.x >> 6] = s;
@@ -646,24 +642,20 @@ __global__ __launch_bounds__(kVecRows) void unit_norm_kernel(int n, double* __re
 }
 
 // x += Z y (k columns)
-template <typename T>
-__global__ void add_zy_kernel(const T* __restrict__ Z, size_t ldz, int n, int k, const T* __restrict__ y,
-                              T* __restrict__ x) {
+__global__ void add_zy_kernel(const double* __restrict__ Z, size_t ldz, int n, int k, const double* __restrict__ y,
+                              double* __restrict__ x) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  T a = x[i];
+  double a = x[i];
   for (int j = 0; j < k; ++j) a += Z[(size_t)j * ldz + i] * y[j];
   x[i] = a;
 }
 
-// y = x * s where s = scal_num / *scal_den (device scalars; den null: 1)
-template <typename T>
-__global__ void scale_kernel(int n, const T* __restrict__ x, T* __restrict__ y, const T* __restrict__ den, T num,
-                             int recip) {
+// y = x / *den
+__global__ void scale_kernel(int n, const double* __restrict__ x, double* __restrict__ y,
+                             const double* __restrict__ den) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const T d = den ? *den : (T)1;
-  y[i] = recip ? x[i] * (num / d) : x[i] * (num * d);
+  if (i < n) y[i] = x[i] * (1.0 / *den);
 }
 
 // r = b - y
@@ -779,7 +771,7 @@ static int inner_solve(IterWork& w, const GmresSetup& g, const double* v, double
   const OrthoWork o{w.part1, w.part2, w.h1, w.inv};
   const dim3 blk(kVecRows), grd(vec_groups(n));
   const bool learned = g.precond == kIterMixedLearned;
-  hipLaunchKernelGGL((krylov_start_kernel<double, float>), grd, blk, 0, s, n, v, V, w.partn);
+  hipLaunchKernelGGL(krylov_start_kernel, grd, blk, 0, s, n, v, V, w.partn);
   for (int j = 0; j < its; ++j) {
     float* Vj = V + (size_t)j * ld;
     float* Zj = Zs + (size_t)j * ld;
@@ -923,7 +915,7 @@ int gmres_solve(IterWork& w, const GmresSetup& g, const double* b, double* x, do
   const dim3 blk(256), grd((n + 255) / 256);
   auto kx = [&](const double* in, double* out) { return apply_k<double>(*g.L, g.M, g.ld, in, out, kw, s); };
   auto norm = [&](const double* v, double* out) -> int {
-    hipLaunchKernelGGL(multi_dot_kernel<double>, dim3(1), blk, 0, s, v, ld, n, v, out);
+    hipLaunchKernelGGL(squared_norm_kernel, dim3(1), blk, 0, s, n, v, out);
     RSD_HIP(hipGetLastError());
     return RSD_OK;
   };
@@ -968,7 +960,7 @@ int gmres_solve(IterWork& w, const GmresSetup& g, const double* b, double* x, do
     double* hb = w.h + (m + 2);
     w.hh[1] = beta;
     RSD_HIP(hipMemcpyAsync(hb, w.hh + 1, sizeof(double), hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL(scale_kernel<double>, grd, blk, 0, s, n, (const double*)r, w.V, (const double*)hb, 1.0, 1);
+    hipLaunchKernelGGL(scale_kernel, grd, blk, 0, s, n, (const double*)r, w.V, (const double*)hb);
     std::fill(gg.begin(), gg.end(), 0.0);
     gg[0] = beta;
     int k = 0;
@@ -1027,7 +1019,7 @@ int gmres_solve(IterWork& w, const GmresSetup& g, const double* b, double* x, do
     }
     if (k > 0) {
       RSD_HIP(hipMemcpyAsync(w.h, yy.data(), k * sizeof(double), hipMemcpyHostToDevice, s));
-      hipLaunchKernelGGL(add_zy_kernel<double>, grd, blk, 0, s, (const double*)w.Z, ld, n, k, (const double*)w.h, x);
+      hipLaunchKernelGGL(add_zy_kernel, grd, blk, 0, s, (const double*)w.Z, ld, n, k, (const double*)w.h, x);
       RSD_HIP(hipGetLastError());
       RSD_HIP(hipStreamSynchronize(s));  // w.h is reused as the next step's scratch
     }

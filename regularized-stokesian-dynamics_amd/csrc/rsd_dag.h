@@ -4,13 +4,14 @@
 //
 // Ticket 0 is the walker; tickets 1 .. dag_tickets() are the lower tiles (i,j)
 // of nt block columns, or, with macro tasks, 2x2 blocks of them; behind them
-// come X = inv(L_S)'s tiles, when a launch forms it.
+// come X = inv(L_S)'s tiles, when a launch forms it.  Which tile a ticket is
+// stands in rsd_dag_tile.inc and rsd_dag_x.inc.
 #pragma once
 
 #if defined(__HIPCC__) || defined(__HIP__)
-#define RSD_DAG_HD __host__ __device__ __forceinline__
+#define RSD_DAG_HD __host__ __device__
 #else
-#define RSD_DAG_HD inline
+#define RSD_DAG_HD
 #endif
 
 namespace rsd {
@@ -38,7 +39,7 @@ constexpr int kMacroTiles = 136;
 // default, one at a time each.
 constexpr int kDagBeside = 19;
 
-RSD_DAG_HD int dag_early(int nt, int c) { return c < nt ? (kEarly < nt - c ? kEarly : nt - c) : 0; }
+RSD_DAG_HD inline int dag_early(int nt, int c) { return c < nt ? (kEarly < nt - c ? kEarly : nt - c) : 0; }
 
 // Ticket order with macro tasks, per pair J of block columns: the early tiles
 // of columns 2J + kAhead and 2J + 1 + kAhead; tile (2J+3, 2J) alone; the macro
@@ -46,7 +47,7 @@ RSD_DAG_HD int dag_early(int nt, int c) { return c < nt ? (kEarly < nt - c ? kEa
 struct MacroCounts {
   int e0, e1, single, macros, last;
 };
-RSD_DAG_HD MacroCounts macro_counts(int nt, int J) {
+RSD_DAG_HD inline MacroCounts macro_counts(int nt, int J) {
   const int m = nt / 2 - (J + 2);
   return {dag_early(nt, 2 * J + kAhead), dag_early(nt, 2 * J + 1 + kAhead), 2 * J + 3 < nt ? 1 : 0, m > 0 ? m : 0,
           (nt & 1) && nt - 1 >= 2 * J + 4 ? 2 : 0};
@@ -62,54 +63,6 @@ inline int dag_tickets(int nt, bool macro) {
     n += k.e0 + k.e1 + k.single + k.macros + k.last;
   }
   return n;
-}
-
-// the tile of ticket t, 1 <= t <= dag_tickets(); macro: the macro task (i, j)
-struct DagTile {
-  int i, j;
-  bool macro;
-};
-RSD_DAG_HD DagTile dag_tile(int nt, bool macro, int t) {
-  int r = t - 1, c0 = 0;
-  for (; c0 < kAhead && c0 < nt; ++c0) {
-    if (r < dag_early(nt, c0)) return {c0 + r, c0, false};
-    r -= dag_early(nt, c0);
-  }
-  if (macro) {
-    for (int J = 0;; ++J) {
-      const MacroCounts k = macro_counts(nt, J);
-      if (r < k.e0 + k.e1) {
-        const int j = 2 * J + kAhead + (r < k.e0 ? 0 : 1);
-        return {j + (r < k.e0 ? r : r - k.e0), j, false};
-      }
-      r -= k.e0 + k.e1;
-      if (r < k.single) return {2 * J + 3, 2 * J, false};
-      r -= k.single;
-      if (r < k.macros) return {J + 2 + r, J, true};
-      r -= k.macros;
-      if (r < k.last) return {nt - 1, 2 * J + r, false};
-      r -= k.last;
-    }
-  }
-  for (int j = 0;; ++j) {
-    const int e = dag_early(nt, j + kAhead), o = nt - j - kEarly > 0 ? nt - j - kEarly : 0;
-    if (r < e) return {j + kAhead + r, j + kAhead, false};
-    r -= e;
-    if (r < o) return {j + kEarly + r, j, false};
-    r -= o;
-  }
-}
-
-// X's tiles (i,j), ns block columns: r = 0 .. ns (ns+1)/2 - 1, the diagonal
-// blocks first, then the others in row order
-RSD_DAG_HD DagTile dag_x_tile(int ns, int r) {
-  if (r < ns) return {r, r, false};
-  int i = 1, j = r - ns;
-  while (j >= i) {
-    j -= i;
-    ++i;
-  }
-  return {i, j, false};
 }
 
 // The persistent workgroups of a launch of nt block columns: at most one per CU,

@@ -1797,9 +1797,7 @@ __device__ __forceinline__ void dag_task(const DagArgs& g, int t, double* __rest
     // (I = s0 + i).  The sum is accumulated transposed, acc = -sum X_kj^T L_Ik^T,
     // from X_kj^T (kept in X's upper block (j,k); X_jj^T in xdT), so that the
     // solve with Dinv_I is tile_trsm's product: X_ij^T = acc Dinv_I^T.
-    const DagTile q = dag_x_tile(ns, r);
-    i = q.i;
-    j = q.j;
+#include "rsd_dag_x.inc"
 #pragma unroll
     for (int bm = 0; bm < 2; ++bm)
 #pragma unroll
@@ -1808,13 +1806,13 @@ __device__ __forceinline__ void dag_task(const DagArgs& g, int t, double* __rest
     T = Terms{j, i, xdT + (size_t)j * 4096, X + 64 * j, A + 64 * I + (size_t)(64 * s0) * ld,
               64, ldx, ld, xf + ns * j, 1, I + nt * s0, nt};
   } else {
-    const DagTile q = dag_tile(nt, MACRO, t);
-    if (MACRO && q.macro) {
-      macro_task(g, q.i, q.j, t, smem);
-      return;
-    }
-    i = q.i;
-    j = q.j;
+#define MACRO_TASK(I, J)               \
+  {                                    \
+    macro_task(g, I, J, t, smem);      \
+    return;                            \
+  }
+#include "rsd_dag_tile.inc"
+#undef MACRO_TASK
     // (the walker takes the tile (j+1,j) transposed)
     const bool tr = i == j + 1;
     const double* src = A + 64 * i + (size_t)(64 * j) * ld;

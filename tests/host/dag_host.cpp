@@ -1,5 +1,6 @@
-// Plays the dataflow Cholesky's order of tasks (csrc/rsd_dag.h) through on the
-// CPU: which tasks finish when a given number of workgroups run at once.
+// Plays the dataflow Cholesky's order of tasks (csrc/rsd_dag.h and the lines that
+// the kernel includes) through on the CPU: which tasks finish when a given number
+// of workgroups run at once.
 //
 // A task is the list of flags that it waits for, in its order, with the flags
 // that it sets between them, as dag_walker, dag_task and macro_task have them.
@@ -18,6 +19,25 @@
 using namespace rsd;
 
 namespace {
+
+// the tile of a ticket; macro: the macro task (i, j)
+struct DagTile {
+  int i, j;
+  bool macro;
+};
+DagTile dag_tile(int nt, bool MACRO, int t) {
+  int i, j;
+#define MACRO_TASK(I, J) return {I, J, true}
+#include "../../regularized-stokesian-dynamics_amd/csrc/rsd_dag_tile.inc"
+#undef MACRO_TASK
+  return {i, j, false};
+}
+DagTile dag_x_tile(int ns, int r) {
+  if (r < ns) return {r, r, false};
+  int i, j;
+#include "../../regularized-stokesian-dynamics_amd/csrc/rsd_dag_x.inc"
+  return {i, j, false};
+}
 
 struct Play {
   int nt, s0, ns;

@@ -1049,7 +1049,9 @@ extern "C" int rsd_ctx_create(rsd_ctx** out, int n, const rsd_step_config* cfg) 
   // HIP deals streams out to its few hardware queues in the order of their
   // creation: the order of the two changes every second context, so that the
   // main streams of a batch take turns at all the queues and not at every other
-  // one (a batch of 12 at width 8: 59.6 -> 56.5 ms)
+  // one (a batch of 12 at width 8: 59.6 -> 56.5 ms).  It is a matter of speed
+  // alone, and holds for contexts made one after the other: streams that the
+  // caller makes in between, or contexts destroyed before, shift the turns.
   static std::atomic<unsigned> created{0};
   const bool side_first = (created.fetch_add(1) >> 1) & 1;
   RSD_HIP(hipStreamCreateWithFlags(side_first ? &c->s2 : &c->s, hipStreamNonBlocking));

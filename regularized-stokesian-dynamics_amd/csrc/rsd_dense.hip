@@ -277,11 +277,6 @@ int gemm_batched(DenseWork& w, const std::vector<GemmDesc>& in, bool ta, bool tb
   return RSD_OK;
 }
 
-// A 64x64 column-major tile (leading dimension ld) into LDS by direct
-// 16-byte global->LDS loads, 1 KB (two columns) per wave instruction, 8 per
-// wave.  Column c of the staged tile holds row m at c*64 + (m ^ 16 (c & 1)):
-// the swap of 16-row halves on odd columns puts the two columns an MFMA
-// operand read touches on different LDS banks.
 // The thread index through an empty asm: address arithmetic derived from it
 // is redone at each call instead of being hoisted out of the persistent
 // Cholesky's ticket loop and held in registers (spilled) across the tasks.
@@ -316,10 +311,14 @@ __device__ __forceinline__ void wt_publish(int* flag, int gen) {
 // the poll (the hardware issues them after the polled value is in)
 __device__ __forceinline__ void wt_seen() { __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront"); }
 
-// A 64x64 tile of the factorization (published by another workgroup) into
-// LDS by direct 16-byte loads at agent scope, past any stale cached copy:
-// a wave's u-th load (of 8) moves columns 16 wave + 2u and 16 wave + 2u + 1;
-// at: the lane's offset into the tile (stage_at), the same for every u.
+// A 64x64 tile of the factorization (published by another workgroup; column-
+// major, leading dimension ld) into LDS by direct 16-byte loads at agent scope,
+// past any stale cached copy, 1 KB (two columns) per wave instruction: a wave's
+// u-th load (of 8) moves columns 16 wave + 2u and 16 wave + 2u + 1; at: the
+// lane's offset into the tile (stage_at), the same for every u.  Column c of
+// the staged tile holds row m at c*64 + (m ^ 16 (c & 1)): the swap of 16-row
+// halves on odd columns puts the two columns an MFMA operand read touches on
+// different LDS banks.
 __device__ __forceinline__ unsigned stage_at(int ld) {
   const int tid = opaque_tid(), lane = tid & 63, wave = tid >> 6;
   return (unsigned)((16 * wave + (lane >> 5)) * ld + 2 * ((lane & 31) ^ ((lane >> 5) << 3)));
@@ -1043,7 +1042,8 @@ struct Terms {
 // scan of one flag pair at a time costs about a microsecond of memory
 // latency per term), and the next scan's loads are in flight during a half.
 // N = 997 (11N = 10967, one factorisation of each order): 16.3 -> 13.6 ms; N = 4096: 981 -> 811 ms; N = 512:
-// 3.22 -> 3.03 ms.  Past N ~ 1000 the tile reads bound it: 64 KB a term, 5.2 TB/s of L2 misses.
+// 3.22 -> 3.03 ms.  From N ~ 550 on the tile reads bound it, 64 KB a term, L2 misses at
+// 5.2 TB/s: 2.4 of an 11N launch's 2.4 ms at N = 576 (1.7 of 1.8 at 512, 0.8 of 1.15 at 400).
 __device__ __forceinline__ void pair_accumulate(v4d (&acc)[2][2], const Terms& T, const int* flags, int gen, int* err,
                                                 double* smem, int* rec, int who) {
   const int kbeg = T.kbeg, kend = T.kend;
@@ -1158,7 +1158,7 @@ __device__ __forceinline__ void pair_accumulate(v4d (&acc)[2][2], const Terms& T
 // A macro task is two block rows by two block columns of the factor, a 128x128
 // tile, accumulated as one: each wave keeps a 64x64 tile of it.  A 64-deep term
 // of four tiles then moves 128 KB into LDS where four single tiles move 256 KB,
-// and past N ~ 700 those reads (L2 misses, 5.2 TB/s) are what bounds the
+// and from N ~ 550 on those reads (L2 misses, 5.2 TB/s) are what bounds the
 // single-tile tasks.  A term is two 32-column halves through two LDS buffers;
 // an 8-step half keeps the matrix cores busy for 8192 cycles, its one barrier
 // is before its last step, and each step's operands are read during the step
